@@ -56,16 +56,18 @@ def gyroid_system():
                    ngrid=[64, 64, 64], chain_step=0.5, group_name="I a -3 d")
 
 
-def kernel_bytes(M, Mk):
+def kernel_bytes(Ms, Mk):
     """Algorithmic HBM bytes per launch of each contour-step kernel for ONE
-    sweep (every array the kernel must read or write, once: FP64 real fields
-    8 B/point, half spectra 16 B/point, factors e1, e2 (M) and k1, k2 (Mk)):
-      step_a : C (Mk) in, q1, e2, e1 (M) in, q (M) out, A, B (Mk) out
-      step_z0: A, B (Mk) in and out, k1, k2 (Mk) in
-      step_c : A, B (Mk) in, e1 (M) in, q1 (M) out, C (Mk) out
-      step_z1: C (Mk) in and out, k2 (Mk) in"""
-    return {"step_a": 32.0 * M + 48.0 * Mk, "step_z0": 80.0 * Mk,
-            "step_c": 16.0 * M + 48.0 * Mk, "step_z1": 40.0 * Mk}
+    sweep (every array the kernel must read or write, once), with Ms stored
+    points of a real field (all N1 N2 N3, or those of the symmetric planes) and
+    Mk half-grid points: FP64 real fields 8 B/point, packed spectra 8 B per
+    stored point, factors e1, e2 (Ms) and k1, k2 (Mk):
+      step_a : spectrum C in, q1, e2, e1 in, q out, A, B out
+      step_z0: A, B in and out, k1, k2 in
+      step_c : A, B in, e1 in, q1 out, C out
+      step_z1: C in and out, k2 in"""
+    return {"step_a": 56.0 * Ms, "step_z0": 32.0 * Ms + 16.0 * Mk,
+            "step_c": 40.0 * Ms, "step_z1": 16.0 * Ms + 8.0 * Mk}
 
 
 def cpu_baseline(g, n_gpu_iter, workdir):
@@ -630,7 +632,7 @@ def main():
     iters = [x.itr for x in results]
     f_fh = S.free_energy_FH()
 
-    M = 64 ** 3
+    M = 64 * 64 * 17               # stored points: Ia-3d's sweeps keep 17 of 64 planes
     Mk = 33 * 64 * 64
     # whole captured sweeps (slot 4): milliseconds and contour steps advanced
     steps_timed = int(n[4])

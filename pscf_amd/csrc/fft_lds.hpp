@@ -18,10 +18,26 @@
 namespace pscf {
 
 // ---------------------------------------------------------------- complex ops
+// a b + c, rounded once on the device.  Where two products are added it is
+// written out which one is fused: kernels that must agree bit for bit (one
+// system alone, many in one launch) may not leave that to the compiler.  Host
+// code (the CPU emulation of the kernels) rounds twice rather than call the C
+// library.
+__device__ __forceinline__ double mad(double a, double b, double c) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_fma(a, b, c);
+#else
+  return a * b + c;
+#endif
+}
 __device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
-  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  return make_double2(mad(a.x, b.x, -(a.y * b.y)), mad(a.x, b.y, a.y * b.x));
+}
+// a * b + c
+__device__ __forceinline__ double2 cfma(double2 a, double2 b, double2 c) {
+  return make_double2(mad(a.x, b.x, mad(-a.y, b.y, c.x)), mad(a.x, b.y, mad(a.y, b.x, c.y)));
 }
 __device__ __forceinline__ double2 cscale(double2 a, double s) { return make_double2(a.x * s, a.y * s); }
 __device__ __forceinline__ double2 cconj(double2 a) { return make_double2(a.x, -a.y); }
@@ -166,8 +182,8 @@ template <int S> struct Dft<5, S> {
     double2 d1 = csub(v[1], v[4]), d2 = csub(v[2], v[3]);
     double2 a1 = make_double2(v[0].x + c1 * t1.x + c2 * t2.x, v[0].y + c1 * t1.y + c2 * t2.y);
     double2 a2 = make_double2(v[0].x + c2 * t1.x + c1 * t2.x, v[0].y + c2 * t1.y + c1 * t2.y);
-    double2 b1 = make_double2(s1 * d1.x + s2 * d2.x, s1 * d1.y + s2 * d2.y);
-    double2 b2 = make_double2(s2 * d1.x - s1 * d2.x, s2 * d1.y - s1 * d2.y);
+    double2 b1 = make_double2(mad(s1, d1.x, s2 * d2.x), mad(s1, d1.y, s2 * d2.y));
+    double2 b2 = make_double2(mad(s2, d1.x, -s1 * d2.x), mad(s2, d1.y, -s1 * d2.y));
     double2 ib1 = cmul_si<S>(b1), ib2 = cmul_si<S>(b2);
     v[0] = cadd(v[0], cadd(t1, t2));
     v[1] = cadd(a1, ib1);
@@ -189,7 +205,7 @@ template <int S> struct Dft<7, S> {
     const double2 d1 = csub(v[1], v[6]), d2 = csub(v[2], v[5]), d3 = csub(v[3], v[4]);
     const double2 x0 = v[0];
     auto lin = [](double2 a, double ca, double2 b, double cb, double2 c, double cc) {
-      return make_double2(ca * a.x + cb * b.x + cc * c.x, ca * a.y + cb * b.y + cc * c.y);
+      return make_double2(mad(cc, c.x, mad(cb, b.x, ca * a.x)), mad(cc, c.y, mad(cb, b.y, ca * a.y)));
     };
     const double2 a1 = cadd(x0, lin(t1, c1, t2, c2, t3, c3));
     const double2 a2 = cadd(x0, lin(t1, c2, t2, c3, t3, c1));

@@ -92,7 +92,7 @@ template <int S> struct Dft<12, S> {
 // 16 = 4 x 4 (Cooley-Tukey): n = 4 n1 + n2, k = k1 + 4 k2,
 // X[k1 + 4 k2] = sum_n2 w4^{n2 k2} w16^{n2 k1} sum_n1 x[4 n1 + n2] w4^{n1 k1}.
 template <int S> __device__ __forceinline__ double2 rot(double2 a, double c, double s) {
-  return make_double2(a.x * c - S * a.y * s, a.y * c + S * a.x * s);   // a e^{S i theta}
+  return make_double2(mad(a.x, c, -(S * s) * a.y), mad(a.y, c, (S * s) * a.x));   // a e^{S i theta}
 }
 template <int S> struct Dft<16, S> {
   static __device__ __forceinline__ void run(double2* v) {
@@ -177,10 +177,12 @@ constexpr int pow2ceil(int n) {
   return p;
 }
 
-template <int N> struct Line {
-  static constexpr int P = line_plan(N).p;
-  static constexpr int Q = line_plan(N).q;
-  static_assert(P > 0 && P * Q == N, "no register line plan for this length");
+// A line of N points on PP threads (default: the length's plan).
+template <int LEN, int PP = line_plan(LEN).p> struct Line {
+  static constexpr int N = LEN;
+  static constexpr int P = PP;
+  static constexpr int Q = N / P;
+  static_assert(P > 0 && P * Q == N && dft_ok(P) && dft_ok(Q), "no register line plan for this length");
   static constexpr int U = (Q + P - 1) / P;       // rounds of layout B
   // every thread holds a point set in every round of layout B (P divides
   // Q); otherwise only the threads t + P u < Q do (all of t < Q when P > Q)
@@ -189,8 +191,9 @@ template <int N> struct Line {
   // line always sit in one wavefront (lanes P..PS-1 of a slot idle)
   static constexpr int PS = pow2ceil(P);
   static_assert(PS <= 64, "a line must fit in one wavefront");
-  // exchange-buffer words of one line with the thread-fastest padding
-  static constexpr int PADW = N + N / (P < Q ? P : Q) + 1;
+  // index of layout-B point (u, k2) of thread t, and whether t holds round u
+  static __device__ __forceinline__ int at(int t, int u, int k2) { return t + P * u + Q * k2; }
+  static __device__ __forceinline__ bool has(int t, int u) { return FULLB || t + P * u < Q; }
 };
 
 // The threads of a line are lanes of one wavefront, which execute in
@@ -204,85 +207,158 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// the value of lane ^ 8: a DPP rotation by half a row of 16 lanes, no LDS.
+// Called by every lane of the wavefront.
+__device__ __forceinline__ double lane_swap(double v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, 0x128, 0xF, 0xF, true);          // row_ror:8
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0x128, 0xF, 0xF, true);
+  return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
+#else
+  return __shfl_xor(v, 8, 64);
+#endif
+}
+__device__ __forceinline__ double2 lane_swap(double2 v) { return make_double2(lane_swap(v.x), lane_swap(v.y)); }
+
 template <int S> __device__ __forceinline__ double2 twid(const double2* tw, int m) {
   double2 w = tw[m];
   if (S > 0) w.y = -w.y;
   return w;
 }
 
-// Layout A -> layout B, DFT of sign S.  eoff(i): exchange slot of element i
-// (i = k1 P + t on write, (t + P u) P + tt on read) of this thread's line;
-// a line's slots are its own, so only its wavefront touches them.  The
-// caller separates other uses of the same LDS words by workgroup barriers.
+// The twiddles of a line's two transforms, w_N^{t k1} (line_fwd) and
+// w_N^{n1 (t + P u)} (line_inv), read from a table in LDS:
+template <class L> struct TwTable {
+  const double2* tw;
+  template <int S> __device__ __forceinline__ double2 f(int t, int k1) const {
+    return twid<S>(tw, (t * k1) % L::N);
+  }
+  template <int S> __device__ __forceinline__ double2 i(int t, int u, int n1) const {
+    return twid<S>(tw, (n1 * (t + L::P * u)) % L::N);
+  }
+};
+// or held in registers by the thread (a thread's t never changes), which
+// frees a line transform of a third of its LDS reads.  INV: line_inv's too.
+// COUNT complex values.
+template <class L, bool INV> struct TwRegs {
+  static constexpr int P = L::P, Q = L::Q, U = L::U;
+  static constexpr bool SHARED = P == Q;      // both transforms use the same values
+  static constexpr bool OWN = INV && !SHARED;
+  static constexpr int COUNT = Q - 1 + (OWN ? U * (P - 1) : 0);
+  double2 wf[Q], wi[OWN ? U : 1][OWN ? P : 1];
+  __device__ __forceinline__ void load(const double2* __restrict__ g, int t) {
+#pragma unroll
+    for (int k1 = 1; k1 < Q; ++k1) wf[k1] = g[(t * k1) % L::N];
+    if constexpr (OWN) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int n1 = 1; n1 < P; ++n1) wi[u][n1] = g[(n1 * (t + P * u)) % L::N];
+    }
+  }
+  template <int S> __device__ __forceinline__ double2 f(int, int k1) const { return twid<S>(wf, k1); }
+  template <int S> __device__ __forceinline__ double2 i(int, int u, int n1) const {
+    if constexpr (SHARED) return twid<S>(wf, n1);
+    else return twid<S>(wi[u], n1);
+  }
+};
+
 template <bool WAVE> __device__ __forceinline__ void line_sync() {
   if constexpr (WAVE) wave_sync();
   else __syncthreads();
 }
 
-template <int N, int S, bool WAVE = true, class EOff>
-__device__ __forceinline__ void line_fwd(double2 (&a)[Line<N>::Q], double2 (&b)[Line<N>::U][Line<N>::P],
-                                         double2* E, EOff eoff, int t, const double2* tw, bool active) {
-  constexpr int P = Line<N>::P, Q = Line<N>::Q, U = Line<N>::U;
-  line_sync<WAVE>();                // the line's earlier reads of its slots are done
-  if (active) {
-    Dft<Q, S>::run(a);
-    if (P > 1) {
+// The two transforms for M lines per thread at once.
+//
+// Layout A -> layout B, DFT of sign S.  eoff(m, i): exchange slot of element
+// i of line m (i = k1 P + t on write, (t + P u) P + tt on read); a line's
+// slots are its own, so only its threads touch them.  The caller separates
+// other uses of the same LDS words by workgroup barriers.
+template <class L, int S, int M, bool WAVE = true, class EOff, class Tw>
+__device__ __forceinline__ void line_fwd(double2 (&a)[M][L::Q], double2 (&b)[M][L::U][L::P], double2* E,
+                                         EOff eoff, int t, const Tw& tw, bool active) {
+  constexpr int P = L::P, Q = L::Q, U = L::U;
+  if constexpr (P == 1) {           // one thread per line: no exchange
+    if (active) {
 #pragma unroll
-      for (int k1 = 1; k1 < Q; ++k1) a[k1] = cmul(a[k1], twid<S>(tw, (t * k1) % N));
-    }
+      for (int m = 0; m < M; ++m) {
+        Dft<Q, S>::run(a[m]);
 #pragma unroll
-    for (int k1 = 0; k1 < Q; ++k1) E[eoff(k1 * P + t)] = a[k1];
-  }
-  line_sync<WAVE>();
-  if (active) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k1 = t + P * u;
-      if (Line<N>::FULLB || k1 < Q) {
-#pragma unroll
-        for (int tt = 0; tt < P; ++tt) b[u][tt] = E[eoff(k1 * P + tt)];
-        Dft<P, S>::run(b[u]);
+        for (int k1 = 0; k1 < Q; ++k1) b[m][k1][0] = a[m][k1];
       }
     }
+    return;
   }
-}
-
-// Layout B -> layout A, DFT of sign S.  eoff(i): exchange slot of element i
-// (i = n1 Q + k1 on write, t Q + k1 on read); slots as in line_fwd.
-template <int N, int S, bool WAVE = true, class EOff>
-__device__ __forceinline__ void line_inv(double2 (&b)[Line<N>::U][Line<N>::P], double2 (&a)[Line<N>::Q],
-                                         double2* E, EOff eoff, int t, const double2* tw, bool active) {
-  constexpr int P = Line<N>::P, Q = Line<N>::Q, U = Line<N>::U;
+  line_sync<WAVE>();                // the lines' earlier reads of their slots are done
+  if (active) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      Dft<Q, S>::run(a[m]);
+#pragma unroll
+      for (int k1 = 1; k1 < Q; ++k1) a[m][k1] = cmul(a[m][k1], tw.template f<S>(t, k1));
+#pragma unroll
+      for (int k1 = 0; k1 < Q; ++k1) E[eoff(m, k1 * P + t)] = a[m][k1];
+    }
+  }
   line_sync<WAVE>();
   if (active) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k1 = t + P * u;
-      if (Line<N>::FULLB || k1 < Q) {
-        Dft<P, S>::run(b[u]);
+    for (int m = 0; m < M; ++m)
 #pragma unroll
-        for (int n1 = 0; n1 < P; ++n1) {
-          double2 v = b[u][n1];
-          if (Q > 1 && n1 > 0) v = cmul(v, twid<S>(tw, (n1 * k1) % N));
-          E[eoff(n1 * Q + k1)] = v;
+      for (int u = 0; u < U; ++u)
+        if (L::has(t, u)) {
+          const int k1 = t + P * u;
+#pragma unroll
+          for (int tt = 0; tt < P; ++tt) b[m][u][tt] = E[eoff(m, k1 * P + tt)];
+          Dft<P, S>::run(b[m][u]);
         }
+  }
+}
+
+// Layout B -> layout A, DFT of sign S.  eoff(m, i): exchange slot of element
+// i of line m (i = n1 Q + k1 on write, t Q + k1 on read); slots as in line_fwd.
+template <class L, int S, int M, bool WAVE = true, class EOff, class Tw>
+__device__ __forceinline__ void line_inv(double2 (&b)[M][L::U][L::P], double2 (&a)[M][L::Q], double2* E,
+                                         EOff eoff, int t, const Tw& tw, bool active) {
+  constexpr int P = L::P, Q = L::Q, U = L::U;
+  if constexpr (P == 1) {
+    if (active) {
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+#pragma unroll
+        for (int k1 = 0; k1 < Q; ++k1) a[m][k1] = b[m][k1][0];
+        Dft<Q, S>::run(a[m]);
       }
     }
+    return;
   }
   line_sync<WAVE>();
   if (active) {
 #pragma unroll
-    for (int k1 = 0; k1 < Q; ++k1) a[k1] = E[eoff(t * Q + k1)];
-    Dft<Q, S>::run(a);
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (L::has(t, u)) {
+          const int k1 = t + P * u;
+          Dft<P, S>::run(b[m][u]);
+#pragma unroll
+          for (int n1 = 0; n1 < P; ++n1) {
+            double2 v = b[m][u][n1];
+            if (Q > 1 && n1 > 0) v = cmul(v, tw.template i<S>(t, u, n1));
+            E[eoff(m, n1 * Q + k1)] = v;
+          }
+        }
   }
-}
-
-// index of layout-B point (u, k2) of thread t
-template <int N> __device__ __forceinline__ int lineB_idx(int t, int u, int k2) {
-  return t + Line<N>::P * u + Line<N>::Q * k2;
-}
-template <int N> __device__ __forceinline__ bool lineB_has(int t, int u) {
-  return Line<N>::FULLB || t + Line<N>::P * u < Line<N>::Q;
+  line_sync<WAVE>();
+  if (active) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+#pragma unroll
+      for (int k1 = 0; k1 < Q; ++k1) a[m][k1] = E[eoff(m, t * Q + k1)];
+      Dft<Q, S>::run(a[m]);
+    }
+  }
 }
 
 }  // namespace pscf

@@ -114,22 +114,44 @@ __global__ void __launch_bounds__(NTA) k_kgrid_to_basis(const double2* __restric
 }
 
 // ----------------------------------------------------------------------------
-// make_propg (src/step_mod.f90:109-129) for one block
+// make_propg (src/step_mod.f90:109-129) for one block: omega on the grid, the
+// factors in the sweeps' packed orders (unpack_index, unpack_kindex; mk
+// z_factors).
 // ----------------------------------------------------------------------------
 __global__ void __launch_bounds__(NTA) k_make_propg(double ds, double b, const double* __restrict__ ksq,
                                                     long mk, const double* __restrict__ omega, long m,
-                                                    double* __restrict__ e1, double* __restrict__ e2,
-                                                    double* __restrict__ k1, double* __restrict__ k2) {
+                                                    int n1, int n2, int zw, double rM, double* __restrict__ e1,
+                                                    double* __restrict__ e2, double* __restrict__ k1,
+                                                    double* __restrict__ k2) {
   const double lap = ds * (b * b) / 6.0;
   const double pot = ds / 2.0;
-  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < m; i += (long)gridDim.x * NTA) {
+  const double norm = (n2 > 1 ? 2.0 : 1.0) * rM;    // see task_k1
+  const long n = m > mk ? m : mk;
+  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < n; i += (long)gridDim.x * NTA) {
     if (i < mk) {
-      k1[i] = exp(-(lap * ksq[i]));
-      k2[i] = exp(-(lap / 2.0 * ksq[i]));
+      const long g = unpack_kindex(i, n1, n2, zw);
+      const double k = g < 0 ? 0.0 : ksq[g];
+      k1[i] = exp(-(lap * k)) / norm;
+      k2[i] = exp(-(lap / 2.0 * k)) / norm;
     }
-    e1[i] = exp(-(pot * omega[i]));
-    e2[i] = exp(-(pot / 2.0 * omega[i]));
+    if (i < m) {
+      const double w = omega[unpack_index(i, n1, n2)];
+      e1[i] = exp(-(pot * w));
+      e2[i] = exp(-(pot / 2.0 * w));
+    }
   }
+}
+
+// nf fields (stride m each) between the grid order and the sweeps' packed order
+__global__ void __launch_bounds__(NTA) k_unpack(const double* __restrict__ packed, long m, int nf, int n1,
+                                                int n2, double* __restrict__ grid) {
+  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < m * nf; i += (long)gridDim.x * NTA)
+    grid[i / m * m + unpack_index(i % m, n1, n2)] = packed[i];
+}
+__global__ void __launch_bounds__(NTA) k_pack(const double* __restrict__ grid, long m, int nf, int n1, int n2,
+                                              double* __restrict__ packed) {
+  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < m * nf; i += (long)gridDim.x * NTA)
+    packed[i] = grid[i / m * m + unpack_index(i % m, n1, n2)];
 }
 
 // ----------------------------------------------------------------------------
@@ -153,11 +175,14 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
   return r;
 }
 
-__global__ void __launch_bounds__(NTA) k_partial_sum(const double* __restrict__ x, long n,
-                                                     double* __restrict__ part) {
+// (a contour point's n values on planes of `plane` points each, weighted where
+// a stored plane stands for several)
+__global__ void __launch_bounds__(NTA) k_partial_sum(const double* __restrict__ x, long n, int sym, int n3,
+                                                     long plane, double* __restrict__ part) {
   __shared__ double red[NTA];
   double acc = 0.0;
-  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < n; i += (long)gridDim.x * NTA) acc += x[i];
+  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < n; i += (long)gridDim.x * NTA)
+    acc += sym ? x[i] * sym_weight(sym, n3, (int)(i / plane)) : x[i];
   const double s = block_sum(acc, red);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
@@ -201,7 +226,8 @@ __global__ void __launch_bounds__(NTA) k_solvent_rho(const double* __restrict__ 
 // Simpson contour integration of one chain (src/scf_mod.fp.f90:362-424, 212-218):
 //   rho_b = ds_b/3 [qf qr(ibgn) + qf qr(iend) + 4 sum_odd + 2 sum_even]
 //   rho_grid(monomer_b) += phi * rho_b / N / Q
-// in the reference's summation order per point.
+// in the reference's summation order per point; q is packed (kernels.hpp), m
+// stored points, rho_grid in grid order, mg points per monomer.
 // ----------------------------------------------------------------------------
 struct SimpsonArgs {
   int nblk;
@@ -213,13 +239,14 @@ struct SimpsonArgs {
 };
 
 __global__ void __launch_bounds__(NTA) k_simpson(const double* __restrict__ qf,
-                                                 const double* __restrict__ qr, long m,
+                                                 const double* __restrict__ qr, long m, long mg,
                                                  SimpsonArgs a, const double* __restrict__ Qp,
-                                                 const double* __restrict__ phimu,
+                                                 const double* __restrict__ phimu, int n1, int n2,
                                                  double* __restrict__ rho_grid) {
   const double Q = Qp[0];
   const double phi = a.ensemble == 1 ? Q * exp(phimu[1]) : phimu[0];
   for (long r = blockIdx.x * (long)NTA + threadIdx.x; r < m; r += (long)gridDim.x * NTA) {
+    const long g = unpack_index(r, n1, n2);
     for (int b = 0; b < a.nblk; ++b) {
       const int ibgn = a.bnd[b], iend = a.bnd[b + 1];
       double acc = qf[(long)ibgn * m + r] * qr[(long)ibgn * m + r];
@@ -230,8 +257,8 @@ __global__ void __launch_bounds__(NTA) k_simpson(const double* __restrict__ qf,
         acc = acc + qf[(long)jj * m + r] * qr[(long)jj * m + r] * 2.0;
       acc = acc * a.ds[b] / 3.0;
       acc = acc / a.chain_length / Q;
-      double* rg = rho_grid + (long)a.monomer[b] * m;
-      rg[r] = rg[r] + phi * acc;
+      double* rg = rho_grid + (long)a.monomer[b] * mg;
+      rg[g] = rg[g] + phi * acc;
     }
   }
 }
@@ -265,12 +292,16 @@ __global__ void __launch_bounds__(NTA) k_stress_dots(const double* __restrict__ 
 // ----------------------------------------------------------------------------
 __global__ void __launch_bounds__(NTA) k_partial_qlogq(const double* __restrict__ qf,
                                                        const double* __restrict__ qr, int use_qf,
-                                                       long n, double* __restrict__ part) {
+                                                       long n, int sym, int n3, long plane,
+                                                       double* __restrict__ part) {
   __shared__ double red[NTA];
   double acc = 0.0;
   for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < n; i += (long)gridDim.x * NTA) {
     const double a = qf[i], b = qr[i];
-    if (a > 0.0 && b > 0.0) acc += a * b * log(use_qf ? a : b);
+    if (a > 0.0 && b > 0.0) {
+      const double v = a * b * log(use_qf ? a : b);
+      acc += sym ? v * sym_weight(sym, n3, (int)(i / plane)) : v;
+    }
   }
   const double s = block_sum(acc, red);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
@@ -290,7 +321,7 @@ __global__ void __launch_bounds__(NTA) k_simpson_lam(const double* __restrict__ 
   __shared__ double red[NTA];
   const int b = blockIdx.y;
   const int ibgn = a.bnd[b], iend = a.bnd[b + 1];
-  const double* lm = lam + (long)a.monomer[b] * m;
+  const double* lm = lam + (long)a.monomer[b] * m;    // packed order, as q
   double tot = 0.0;
   for (long r = blockIdx.x * (long)NTA + threadIdx.x; r < m; r += (long)gridDim.x * NTA) {
     double acc = qf[(long)ibgn * m + r] * qr[(long)ibgn * m + r];
@@ -327,17 +358,19 @@ __global__ void __launch_bounds__(NTA) k_simpson_seg(const double* __restrict__ 
 }
 
 // rho_grid(monomer_b) += phi / (N Q) * blk_b for every block of a chain
-__global__ void __launch_bounds__(NTA) k_block_rho(const double* __restrict__ blk, long m,
+__global__ void __launch_bounds__(NTA) k_block_rho(const double* __restrict__ blk, long m, long mg,
                                                    SimpsonArgs a, const double* __restrict__ Qp,
-                                                   const double* __restrict__ phimu,
+                                                   const double* __restrict__ phimu, int n1, int n2,
                                                    double* __restrict__ rho_grid) {
   const double Q = Qp[0];
   const double phi = a.ensemble == 1 ? Q * exp(phimu[1]) : phimu[0];
-  for (long r = blockIdx.x * (long)NTA + threadIdx.x; r < m; r += (long)gridDim.x * NTA)
+  for (long r = blockIdx.x * (long)NTA + threadIdx.x; r < m; r += (long)gridDim.x * NTA) {
+    const long g = unpack_index(r, n1, n2);
     for (int b = 0; b < a.nblk; ++b) {
-      double* rg = rho_grid + (long)a.monomer[b] * m;
-      rg[r] = rg[r] + phi * (blk[(long)b * m + r] / a.chain_length / Q);
+      double* rg = rho_grid + (long)a.monomer[b] * mg;
+      rg[g] = rg[g] + phi * (blk[(long)b * m + r] / a.chain_length / Q);
     }
+  }
 }
 
 // workgroup partials of sum x*y
@@ -351,10 +384,11 @@ __global__ void __launch_bounds__(NTA) k_partial_dot(const double* __restrict__ 
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// y += x (n values)
-__global__ void __launch_bounds__(NTA) k_axpy1(const double* __restrict__ x, long n,
+// y += x (n values), x in the sweeps' packed order, y in grid order
+__global__ void __launch_bounds__(NTA) k_axpy1(const double* __restrict__ x, long n, int n1, int n2,
                                                double* __restrict__ y) {
-  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < n; i += (long)gridDim.x * NTA) y[i] += x[i];
+  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < n; i += (long)gridDim.x * NTA)
+    y[unpack_index(i, n1, n2)] += x[i];
 }
 
 // Cell derivative of a |k|^2 gradient: for each cell parameter p (blockIdx.y),
@@ -379,6 +413,43 @@ __global__ void __launch_bounds__(NTA) k_dksq_dot(GeomArgs g, const double* __re
   }
   const double s = block_sum(acc, red);
   if (threadIdx.x == 0) part[(long)p * gridDim.x + blockIdx.x] = s;
+}
+
+// nf grid fields whose stored planes (symmetric planes, kernels.hpp) are set:
+// the others from them
+__global__ void __launch_bounds__(NTA) k_sym_expand(double* __restrict__ f, int nf, int sym, int n1, int n2,
+                                                    int n3) {
+  const long m = (long)n1 * n2 * n3, m0 = (long)n1 * n2 * sym_planes(sym, n3);
+  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < (m - m0) * nf; i += (long)gridDim.x * NTA) {
+    double* g = f + i / (m - m0) * m;
+    const long p = m0 + i % (m - m0);
+    g[p] = g[sym_point(sym, n1, n2, n3, p)];
+  }
+}
+// one packed contour point on its stored planes -> the whole field, in packed
+// (pack) or grid order
+__global__ void __launch_bounds__(NTA) k_sym_point(const double* __restrict__ q, long qs, int sym, int n1, int n2,
+                                                   int n3, int pack, double* __restrict__ out, long os) {
+  const long m = (long)n1 * n2 * n3;
+  q += blockIdx.y * qs;
+  out += blockIdx.y * os;
+  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < m; i += (long)gridDim.x * NTA) {
+    const long g = pack ? unpack_index(i, n1, n2) : i;
+    out[i] = q[pack_index(sym_point(sym, n1, n2, n3, g), n1, n2)];
+  }
+}
+// flag[0] = epoch if a field has a value further than tol from that of its
+// stored point: it is not symmetric
+__global__ void __launch_bounds__(NTA) k_sym_check(const double* __restrict__ f, int nf, int sym, int n1, int n2,
+                                                   int n3, double tol, double epoch, double* __restrict__ flag) {
+  const long m = (long)n1 * n2 * n3, m0 = (long)n1 * n2 * sym_planes(sym, n3);
+  bool bad = false;
+  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < (m - m0) * nf; i += (long)gridDim.x * NTA) {
+    const double* g = f + i / (m - m0) * m;
+    const long p = m0 + i % (m - m0);
+    bad = bad || !(fabs(g[p] - g[sym_point(sym, n1, n2, n3, p)]) <= tol);
+  }
+  if (bad) flag[0] = epoch;
 }
 
 // constant fill

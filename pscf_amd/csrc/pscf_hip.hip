@@ -137,15 +137,16 @@ const double2* twiddles(int n) {
 }
 
 // ------------------------------------------------------- kernel dispatch
-using StepPlaneFn = void (*)(const StepTask*, int, int, const double2*, const double2*);
-using StepZFn = void (*)(const StepTask*, int, int, int, const double2*);
+using StepPlaneFn = void (*)(const StepTask*, int, const double2*, const double2*);
+using StepZFn = void (*)(const StepTask*, int, int, int, const double2*, const double2*);
 using R2CFn = void (*)(const double*, long, double2*, long, const double2*, const double2*,
                        const int*, int);
 using C2RFn = void (*)(const double2*, long, double*, long, double, const double2*, const double2*);
 using R2CColsFn = void (*)(const double*, const double*, long, double2*, long, const double2*,
-                           const double2*, const int*, int, int);
+                           const double2*, const int*, int);
 using ZfftFn = void (*)(double2*, long, int, const double2*);
-using ZColsFn = void (*)(double2*, long, long, const double2*);
+using ZColsFn = void (*)(int, const double2*, long, int, double2*, long, int, int, const int2*, const int2*,
+                         const double2*, const double2*);
 using C2CFn = void (*)(double2*, long, const double2*, const double2*);
 
 struct PlaneSet {
@@ -153,9 +154,9 @@ struct PlaneSet {
   int nt_step = 0;            // workgroup size of the step plane kernels
   int ajobs = 0;              // workgroups per plane of k_step_a (0: by occupancy)
   size_t lds_step = 0;        // LDS bytes of a step plane workgroup
-  StepPlaneFn a1 = nullptr;   // k_step_a, one workgroup per plane
-  StepPlaneFn a = nullptr, c = nullptr;
-  StepPlaneFn c_wide = nullptr;   // k_step_c with shared exchange/plane LDS (wide launches)
+  // [adjoint sweeps]: k_step_a with one and two workgroups per plane, k_step_c,
+  // and k_step_c with shared exchange/plane LDS (wide launches)
+  StepPlaneFn a1[2] = {}, a[2] = {}, c[2] = {}, c_wide[2] = {};
   R2CFn r2c = nullptr;
   R2CColsFn r2c_cols = nullptr;   // register-line XY pass of scf_stress's transforms
   C2RFn c2r = nullptr;
@@ -164,8 +165,9 @@ struct PlaneSet {
 struct ZSet {
   int nt_half = 0, nt_full = 0;   // workgroup sizes (zcol_nt for N1/2+1 and N1 wide rows)
   int nt_step = 0;                // workgroup size of the step z kernel
-  int zw = 1;                     // its half-spectrum columns per workgroup
-  StepZFn z = nullptr;
+  int nt_cols = 0;                // of the stress transform's z kernel
+  int zw = 1;                     // their column slots and columns per workgroup
+  StepZFn z[3] = {};              // [Z_PLAIN, Z_ADJ, Z_SYM]
   ZfftFn half_f = nullptr, half_i = nullptr, full_f = nullptr, full_i = nullptr;
   ZColsFn cols_f = nullptr;       // register-line forward z pass of scf_stress's spectra
 };
@@ -181,12 +183,17 @@ PlaneSet make_plane() {
   s.nt_step = StepPlane<A, B>::NT;
   s.ajobs = plan_ajobs(A);
   s.lds_step = StepPlane<A, B>::LDS;
-  s.a = k_step_a<A, B, false>;
-  s.a1 = k_step_a<A, B, true>;
-  s.c = k_step_c<A, B>;
+  s.a[0] = k_step_a<A, B, false, false>;
+  s.a[1] = k_step_a<A, B, false, true>;
+  s.a1[0] = k_step_a<A, B, true, false>;
+  s.a1[1] = k_step_a<A, B, true, true>;
+  s.c[0] = k_step_c<A, B, false>;
+  s.c[1] = k_step_c<A, B, true>;
   // at most 128 VGPRs where that costs no spills and frees a resident
   // workgroup (edges 48 to 64; lines of 40 points spill under the cap)
-  s.c_wide = k_step_c<A, B, 40 * 1024, (A >= 48 && A <= 64 && B >= 48 && B <= 64 ? 4 : 1)>;
+  constexpr int wpe = A >= 48 && A <= 64 && B >= 48 && B <= 64 ? 4 : 1;
+  s.c_wide[0] = k_step_c<A, B, false, 40 * 1024, wpe>;
+  s.c_wide[1] = k_step_c<A, B, true, 40 * 1024, wpe>;
   s.r2c = k_plane_r2c<A, B>;
   s.r2c_cols = k_plane_r2c_cols<A, B>;
   s.c2r = k_plane_c2r<A, B>;
@@ -202,8 +209,11 @@ ZSet make_z() {
   s.nt_half = zcol_nt(A / 2 + 1, C);
   s.nt_full = zcol_nt(A, C);
   s.nt_step = StepZ<C>::NT;
+  s.nt_cols = StepZ<C>::NTC;
   s.zw = StepZ<C>::ZW;
-  s.z = k_step_z<A, C>;
+  s.z[Z_PLAIN] = k_step_z<A, C, Z_PLAIN>;
+  s.z[Z_ADJ] = k_step_z<A, C, Z_ADJ>;
+  if constexpr (C > 1) s.z[Z_SYM] = k_step_z<A, C, Z_SYM>;
   s.half_f = k_zfft<A / 2 + 1, C, -1>;
   s.cols_f = k_zfwd_cols<C>;
   s.half_i = k_zfft<A / 2 + 1, C, +1>;
@@ -276,12 +286,19 @@ int grid_blocks(long n) {
 // ------------------------------------------------------------- geometry
 struct Grid {
   int n1 = 0, n2 = 0, n3 = 0, dim = 0, n1h = 0;
+  int nl = 1;                 // packed rows per plane
   long m = 0, mk = 0;
+  long mc = 0;                // complex words of a packed spectrum
+  long mf = 0;                // reciprocal-space factors of a block (z_factors)
+  // symmetric planes (kernels.hpp): the code (0: none), and what the sweeps
+  // store: np planes, ms points of a real field (mc counts those planes too)
+  int sym = 0, np = 0;
+  long ms = 0;
   const PlaneSet* pl = nullptr;
   const ZSet* zs = nullptr;
   long cus = 0;               // compute units
   long plane_slots = 0;       // plane workgroups resident at once (CUs x LDS fit)
-  const double2 *tw1 = nullptr, *tw2 = nullptr, *tw3 = nullptr;
+  const double2 *tw1 = nullptr, *tw2 = nullptr, *tw3 = nullptr, *twl = nullptr;
 
   // with_tw false: the twiddle tables are left to the caller (no device allocation)
   void init(const int ng[3], int d, bool with_tw = true) {
@@ -294,6 +311,8 @@ struct Grid {
     n1h = n1 / 2 + 1;
     m = (long)n1 * n2 * n3;
     mk = (long)n1h * n2 * n3;
+    nl = n2 > 1 ? n2 / 2 : 1;
+    set_sym(0);
     auto ip = plane_table().find({n1, n2});
     auto iz = z_table().find({n1, n3});
     char buf[160];
@@ -301,6 +320,7 @@ struct Grid {
     REQUIRE(ip != plane_table().end() && iz != z_table().end(), buf);
     pl = &ip->second;
     zs = &iz->second;
+    mf = z_factors(n1, n2, n3, zs->zw);
     int dev = 0, cus = 0, lds_cu = 0;
     HIPCHK(hipGetDevice(&dev));
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -311,34 +331,41 @@ struct Grid {
       tw1 = twiddles(n1);
       tw2 = twiddles(n2);
       tw3 = twiddles(n3);
+      twl = twiddles(nl);
     }
+  }
+
+  void set_sym(int code) {
+    sym = code;
+    np = sym_planes(code, n3);
+    ms = (long)n1 * n2 * np;
+    mc = (long)plane_words(n1, nl) * np;
   }
 
   // step kernels over ntask sweep tasks at launch step j (run_sweeps' order:
   // step_a, step_z kind 0 (2 jobs), step_c (2 jobs), step_z kind 1)
   // With events (t0, t1), the launch records them at the start and the end of
   // the kernel's execution (hipExtLaunchKernelGGL: no launch gaps included).
-  void step_z(const StepTask* tasks, int ntask, int j, int kind, int jobs, hipStream_t s,
+  // adj: the tasks are adjoint or recomputed sweeps
+  void step_z(const StepTask* tasks, int ntask, int j, int kind, int jobs, bool adj, hipStream_t s,
               hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr) const {
-    const long ncol = (long)n1h * n2;
-    const dim3 grid((unsigned)((ncol + zs->zw - 1) / zs->zw), ntask, jobs);
+    const dim3 grid(z_tiles(n1, nl, zs->zw), ntask, jobs);
+    const StepZFn k = zs->z[adj ? Z_ADJ : (sym ? Z_SYM : Z_PLAIN)];
     if (t0)
-      hipExtLaunchKernelGGL(zs->z, grid, dim3(zs->nt_step), 0, s, t0, t1, 0, tasks, j, n2, kind, tw3);
+      hipExtLaunchKernelGGL(k, grid, dim3(zs->nt_step), 0, s, t0, t1, 0, tasks, j, n2, kind, tw2, tw3);
     else
-      hipLaunchKernelGGL(zs->z, grid, dim3(zs->nt_step), 0, s, tasks, j, n2, kind, tw3);
+      hipLaunchKernelGGL(k, grid, dim3(zs->nt_step), 0, s, tasks, j, n2, kind, tw2, tw3);
   }
   // launches that need more than two rounds of resident workgroups take the
   // form whose smaller LDS footprint lets more of them reside on a CU at once
-  // (BCC 64^3, 16 sweeps per launch: 6.5 -> 5.8 us per chain; at 8 sweeps
-  // per launch, two rounds either way, the shared-buffer form is slower)
-  void step_c(const StepTask* tasks, int ntask, int j, hipStream_t s, hipEvent_t t0 = nullptr,
+  void step_c(const StepTask* tasks, int ntask, int j, bool adj, hipStream_t s, hipEvent_t t0 = nullptr,
               hipEvent_t t1 = nullptr) const {
-    const StepPlaneFn k = (long)n3 * ntask * 2 > 2 * plane_slots ? pl->c_wide : pl->c;
+    const StepPlaneFn k = (long)np * ntask * 2 > 2 * plane_slots ? pl->c_wide[adj] : pl->c[adj];
     if (t0)
-      hipExtLaunchKernelGGL(k, dim3(n3, ntask, 2), dim3(pl->nt_step), 0, s, t0, t1, 0, tasks, j, n3,
-                            tw1, tw2);
+      hipExtLaunchKernelGGL(k, dim3(np, ntask, 2), dim3(pl->nt_step), 0, s, t0, t1, 0, tasks, j,
+                            tw1, twl);
     else
-      hipLaunchKernelGGL(k, dim3(n3, ntask, 2), dim3(pl->nt_step), 0, s, tasks, j, n3, tw1, tw2);
+      hipLaunchKernelGGL(k, dim3(np, ntask, 2), dim3(pl->nt_step), 0, s, tasks, j, tw1, twl);
   }
   // real (nb arrays, stride m) -> half spectra (stride mk)
   void r2c(const double* in, double2* out, int nb, hipStream_t s) const {
@@ -347,21 +374,19 @@ struct Grid {
     if (n3 > 1)
       hipLaunchKernelGGL(zs->half_f, dim3(n2, nb), dim3(zs->nt_half), 0, s, out, mk, n2, tw3);
   }
-  // the same transform kept on ncolp columns of every XY half plane (cpos:
-  // half-plane entry -> column position or -1; ncol used, ncolp a multiple of
-  // n1h), out[b][z][c] with stride n3*ncolp, for nb arrays at `in` and, when
-  // in2 is given, nb more at in2 (their outputs after the first nb).  Both
-  // passes run on the step kernels' register lines; the z pass on the ncolp
-  // columns only.
-  void r2c_cols(const double* in, const double* in2, double2* out, int nb, const int* cpos,
-                int ncol, int ncolp, hipStream_t s) const {
-    const long st = (long)n3 * ncolp;
+  // contour points in packed order (nb arrays at `in` and, when in2 is given,
+  // nb more at in2, outputs after the first nb) -> their half spectra on ncol
+  // columns, out[b][z][c]; the XY pass keeps the nin packed columns (cpos:
+  // packed-plane entry -> column or -1) that those are split from (src, cols:
+  // k_zfwd_cols) in `work`.  Both passes run on the step kernels' lines.
+  void r2c_cols(const double* in, const double* in2, double2* work, double2* out, int nb, const int* cpos,
+                int nin, int ncol, const int2* src, const int2* cols, hipStream_t s) const {
     const int sets = in2 ? 2 : 1;
-    hipLaunchKernelGGL(pl->r2c_cols, dim3(n3, nb, sets), dim3(pl->nt_step), 0, s, in, in2, m, out,
-                       st, tw1, tw2, cpos, ncol, ncolp);
-    if (n3 > 1)
-      hipLaunchKernelGGL(zs->cols_f, dim3((unsigned)((ncolp + zs->zw - 1) / zs->zw), nb * sets),
-                         dim3(zs->nt_step), 0, s, out, st, (long)ncolp, tw3);
+    hipLaunchKernelGGL(pl->r2c_cols, dim3(np, nb, sets), dim3(pl->nt_step), 0, s, in, in2, ms, work,
+                       (long)np * nin, tw1, twl, cpos, nin);
+    hipLaunchKernelGGL(zs->cols_f, dim3((unsigned)((ncol + zs->zw - 1) / zs->zw), nb * sets),
+                       dim3(zs->nt_cols), 0, s, sym, work, (long)np * nin, nin, out, (long)n3 * ncol, ncol, n2,
+                       src, cols, tw2, tw3);
   }
   // half spectra -> real, in place on `in` for the z pass
   void c2r(double2* in, double* out, int nb, double scale, hipStream_t s) const {
@@ -427,6 +452,16 @@ bool is_device_pointer(const void* p) {
     return false;
   }
   return a.type == hipMemoryTypeDevice;
+}
+
+// the single block of a one-step task with factors at f (pscf_step_*)
+void one_step_blocks(StepTask& t, const Grid& g, const double* f) {
+  t.nblk = 1;
+  t.bnd[0] = 0;
+  for (int b = 1; b <= MAXBLK; ++b) t.bnd[b] = 1;
+  t.fac = f;
+  t.fm = g.ms;
+  t.fk = g.mf;
 }
 
 // ------------------------------------------------------------ fft plan
@@ -530,12 +565,12 @@ struct System {
   DevBuf<int> star_of_wave, star_invert, wtab, kwave, sconj;
   DevBuf<double2> coeff, scoef;
   DevBuf<long> sidx;
-  // stress transforms keep only the half-spectrum columns (kx, ky) holding a
-  // star's representative wave: ncolp columns (a multiple of N1/2+1, padded
-  // with column 0), their positions in an XY half plane, and per star the
-  // index of its representative in that compact (z, column) layout
-  int ncol = 0, ncolp = 0;
-  DevBuf<int> scpos;             // half-plane entry -> its compact column, or -1
+  // stress transforms keep only the ncol half-spectrum columns (kx, ky)
+  // holding a star's representative wave, and the nin packed columns they are
+  // split from; per star the index of its representative at (z, column)
+  int ncol = 0, nin = 0;
+  DevBuf<int> scpos;             // packed-plane entry -> its position among the nin, or -1
+  DevBuf<int2> ssrc, scolk;      // per column: its two packed positions, its (kx, ky)
   DevBuf<long> sidx_c;
   std::vector<int> h_wave, h_wave_of_star, h_star_of_wave, h_star_invert;
   std::vector<int> h_wtab;   // dense which_wave table (1-based wave, 0: none) over gmin + [0, gext)
@@ -580,6 +615,19 @@ struct System {
   // copies of the system are rebuilt when they change)
   uint64_t gen_basis = 0, gen_start = 0;
   std::unique_ptr<Multi> multi;
+  // symmetric planes of the star basis (code, 0: none; found by detect_sym)
+  // and, per star, a bound of its function's modulus
+  int sym_code = 0;
+  std::vector<double> star_bound;
+  bool no_sym = false;           // store every plane whatever the basis
+  bool sym_bad = false;          // an omega field of this basis was not symmetric
+  double sym_epoch = 0.0;        // density() calls checked so far
+  // the same system with every plane stored, for fields that need not have
+  // the basis's symmetry (density on grids, reverse mode); made when needed.
+  // last: it holds the results of the last density()
+  std::unique_ptr<System> full;
+  uint64_t full_basis = 0, full_start = 0;
+  System* last = nullptr;
   ~System();
   // contour sweeps of one density() captured once as a HIP graph
   int ntask = 0, max_ns = 0;
@@ -649,27 +697,28 @@ void discretize(int nblk, const double* L, double ds0, int order, int* bgn, doub
 }
 
 // ------------------------------------------------------------ reductions
-// out_dev[0] = sum(x[0..n)) * scale (async)
-void dev_sum(const double* x, long n, double scale, double* part, double* out_dev, hipStream_t s) {
-  const int nb = grid_blocks(n) > 512 ? 512 : grid_blocks(n);
-  hipLaunchKernelGGL(k_partial_sum, dim3(nb), dim3(NTA), 0, s, x, n, part);
+// out_dev[0] = scale * sum of a contour point over the whole grid (async)
+void dev_sum(const Grid& g, const double* x, double scale, double* part, double* out_dev, hipStream_t s) {
+  const int nb = grid_blocks(g.ms) > 512 ? 512 : grid_blocks(g.ms);
+  hipLaunchKernelGGL(k_partial_sum, dim3(nb), dim3(NTA), 0, s, x, g.ms, g.sym, g.n3, (long)g.n1 * g.n2, part);
   hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(NTA), 0, s, part, nb, scale, out_dev);
 }
 
 // k_step_a for ntask sweeps: two workgroups per plane (more parallelism)
 // while one per plane would leave CUs idle and two all fit in one round of
 // resident workgroups; else one (a quarter less work).  A plan may force either.
-void launch_step_a(const Grid& g, const StepTask* tasks, int ntask, int j, hipStream_t s,
+void launch_step_a(const Grid& g, const StepTask* tasks, int ntask, int j, bool adj, hipStream_t s,
                    hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr) {
   int aj = g.pl->ajobs;
-  const long planes = (long)g.n3 * ntask;
+  const long planes = (long)g.np * ntask;
   if (aj == 0) aj = (planes < g.cus && 2 * planes <= g.plane_slots) ? 2 : 1;
-  StepPlaneFn k = aj == 1 ? g.pl->a1 : g.pl->a;
-  const dim3 grid(g.n3, ntask, aj);
+  StepPlaneFn k = aj == 1 ? g.pl->a1[adj] : g.pl->a[adj];
+  const dim3 grid(g.np, ntask, aj);
   if (t0)
-    hipExtLaunchKernelGGL(k, grid, dim3(g.pl->nt_step), 0, s, t0, t1, 0, tasks, j, g.n3, g.tw1, g.tw2);
+    hipExtLaunchKernelGGL(k, grid, dim3(g.pl->nt_step), 0, s, t0, t1, 0, tasks, j, g.tw1,
+                          g.twl);
   else
-    hipLaunchKernelGGL(k, grid, dim3(g.pl->nt_step), 0, s, tasks, j, g.n3, g.tw1, g.tw2);
+    hipLaunchKernelGGL(k, grid, dim3(g.pl->nt_step), 0, s, tasks, j, g.tw1, g.twl);
 }
 
 // --------------------------------------------------- contour sweeps
@@ -683,14 +732,14 @@ void run_sweeps(const Grid& g, const StepTask* d_tasks, int ntask, int max_ns, h
   auto t1 = [&] { return ev ? ev[e + 1] : nullptr; };
   auto next = [&] { if (ev) e += 2; };
   for (int j = 0; j <= max_ns; ++j) {
-    launch_step_a(g, d_tasks, ntask, j, s, t0(), t1());
+    launch_step_a(g, d_tasks, ntask, j, false, s, t0(), t1());
     next();
     if (j == max_ns) break;
-    g.step_z(d_tasks, ntask, j, 0, 2, s, t0(), t1());
+    g.step_z(d_tasks, ntask, j, 0, 2, false, s, t0(), t1());
     next();
-    g.step_c(d_tasks, ntask, j, s, t0(), t1());
+    g.step_c(d_tasks, ntask, j, false, s, t0(), t1());
     next();
-    g.step_z(d_tasks, ntask, j, 1, 1, s, t0(), t1());
+    g.step_z(d_tasks, ntask, j, 1, 1, false, s, t0(), t1());
     next();
   }
   HIPCHK(hipGetLastError());
@@ -727,6 +776,56 @@ void ensure_events(System& S, size_t n) {
   }
 }
 
+// The code of the star basis's symmetric planes (kernels.hpp).  An operation
+// r -> W r + t leaves every star function unchanged when the coefficients of
+// its waves obey c(W^T G) = c(G) exp(i G t), W^T G in the same star.
+// Translations z -> z + N3/2 are tried with a = +1 (centring) before a = -1
+// (screw axis), reflections z -> -z with a = -1 (inversion) before +1, each
+// with tau = 0 or half an edge.  Waves whose image lies outside the wave list
+// (on the zone boundary) do not count; every field is checked besides
+// (k_sym_check).
+int detect_sym(const System& S) {
+  const Grid& g = S.g;
+  if (g.dim != 3 || g.n3 % 4 || g.n1 % 2 || g.n2 % 2 || S.no_sym) return 0;
+  const long step = std::max(1, S.nwave / 8192);
+  auto holds = [&](int sz, int a, int tx, int ty, int tz) {
+    long seen = 0;
+    for (long w = 0; w < S.nwave; w += w < 4096 ? 1 : step) {
+      const int* G = &S.h_wave[(size_t)w * 3];
+      const int Gp[3] = {a * G[0], a * G[1], sz * G[2]};
+      long off = 0, mul = 1;
+      bool in = true;
+      for (int d = 0; d < 3; ++d) {
+        const int u = Gp[d] - S.gmin[d];
+        in = in && u >= 0 && u < S.gext[d];
+        off += (long)u * mul;
+        mul *= S.gext[d];
+      }
+      const int v = in ? S.h_wtab[off] : 0;
+      if (v == 0) continue;
+      const double2 c = S.h_coeff[w], cp = S.h_coeff[v - 1];
+      const double sg = ((tx * G[0] + ty * G[1] + tz * G[2]) & 1) ? -1.0 : 1.0;
+      if (S.h_star_of_wave[v - 1] != S.h_star_of_wave[w] || std::fabs(cp.x - sg * c.x) > 1e-10 ||
+          std::fabs(cp.y - sg * c.y) > 1e-10)
+        return false;
+      ++seen;
+    }
+    return seen > 0;
+  };
+  int code = 0, t = 0, r = 0;
+  for (int k = 0; k < 8 && !(code & SYM_T); ++k)
+    if (holds(1, k < 4 ? 1 : -1, k & 1, k >> 1 & 1, 1)) {
+      code |= SYM_T;
+      t = (k < 4 ? 0 : 1) | (k & 1) << 1 | (k >> 1 & 1) << 2;
+    }
+  for (int k = 0; k < 8 && !(code & SYM_R); ++k)
+    if (holds(-1, k < 4 ? -1 : 1, k & 1, k >> 1 & 1, 0)) {
+      code |= SYM_R;
+      r = (k < 4 ? 1 : 0) | (k & 1) << 1 | (k >> 1 & 1) << 2;
+    }
+  return code ? code | t << 2 | r << 5 | (t ^ r) << 8 : 0;
+}
+
 void build_basis_maps(System& S) {
   // dense which_wave table over the bounding box of the wave list
   const int dim = S.g.dim;
@@ -761,6 +860,9 @@ void build_basis_maps(System& S) {
   for (int w = 0; w < S.nwave; ++w) wt[box(&S.h_wave[(size_t)w * dim])] = w + 1;
   S.wtab.upload(wt.data(), wt.size(), S.st.s);
   S.h_wtab = wt;
+  S.star_bound.assign(S.nstar, 0.0);
+  for (int w = 0; w < S.nwave; ++w)
+    S.star_bound[S.h_star_of_wave[w] - 1] += std::hypot(S.h_coeff[w].x, S.h_coeff[w].y);
   // per star: representative wave -> half-grid index (conj if kx > N1/2), coeff
   std::vector<long> sidx(S.nstar);
   std::vector<int> sconj(S.nstar);
@@ -782,23 +884,36 @@ void build_basis_maps(System& S) {
     sidx[s] = kf[0] + (long)S.g.n1h * (kf[1] + (long)S.g.n2 * kf[2]);
   }
   S.sidx.upload(sidx.data(), sidx.size(), S.st.s);
+  // half-spectrum columns (kx, ky) with a representative wave, and the packed
+  // columns (kx, l), (-kx, -l) they are split from
   const long plane = (long)S.g.n1h * S.g.n2;
+  const int nl = S.g.nl, n1 = S.g.n1;
   std::vector<int> cols;
   for (int s = 0; s < S.nstar; ++s) cols.push_back((int)(sidx[s] % plane));
   std::sort(cols.begin(), cols.end());
   cols.erase(std::unique(cols.begin(), cols.end()), cols.end());
-  const int ncol = (int)cols.size();
-  S.ncolp = (ncol + S.g.n1h - 1) / S.g.n1h * S.g.n1h;
+  S.ncol = (int)cols.size();
   std::vector<long> sidx_c(S.nstar);
   for (int s = 0; s < S.nstar; ++s) {
     const int c = (int)(std::lower_bound(cols.begin(), cols.end(), (int)(sidx[s] % plane)) -
                         cols.begin());
-    sidx_c[s] = c + (long)S.ncolp * (sidx[s] / plane);
+    sidx_c[s] = c + (long)S.ncol * (sidx[s] / plane);
   }
-  S.ncol = ncol;
-  std::vector<int> cpos((size_t)plane, -1);
-  for (int c = 0; c < ncol; ++c) cpos[cols[c]] = c;
+  std::vector<int> cpos((size_t)n1 * nl, -1);
+  std::vector<int2> src(S.ncol), colk(S.ncol);
+  for (int c = 0; c < S.ncol; ++c) {
+    const int kx = cols[c] % S.g.n1h, ky = cols[c] / S.g.n1h, l = ky % nl;
+    colk[c] = make_int2(kx, ky);
+    src[c] = make_int2(l * n1 + col_pos(kx, n1), (nl - l) % nl * n1 + col_pos((n1 - kx) % n1, n1));
+    cpos[src[c].x] = cpos[src[c].y] = 0;
+  }
+  S.nin = 0;
+  for (auto& p : cpos)
+    if (p == 0) p = S.nin++;
+  for (auto& p : src) p = make_int2(cpos[p.x], cpos[p.y]);
   S.scpos.upload(cpos.data(), cpos.size(), S.st.s);
+  S.ssrc.upload(src.data(), src.size(), S.st.s);
+  S.scolk.upload(colk.data(), colk.size(), S.st.s);
   S.sidx_c.upload(sidx_c.data(), sidx_c.size(), S.st.s);
   S.sconj.upload(sconj.data(), sconj.size(), S.st.s);
   S.scoef.upload(scoef.data(), scoef.size(), S.st.s);
@@ -976,7 +1091,7 @@ void build_ck_plan(System& S) {
         StepTask t = S.h_tasks[2 * c + d];
         StepTask& o = ht[((size_t)r * nc + c) * 2 + d];
         t.init_one = 0;
-        t.slab = ch.seg.p + (size_t)d * ch.segpts * S.g.m;
+        t.slab = ch.seg.p + (size_t)d * ch.segpts * S.g.ms;
         t.pmap = P.maps.p + P.map_off[((size_t)r * nc + c) * 2 + 0];
         if (lo >= hi) {
           t.skip = 1;
@@ -1003,8 +1118,8 @@ void ck_simpson_rounds(System& S, hipStream_t s) {
   const int nc = S.nchain, K = S.ck_stride;
   for (int c = 0; c < nc; ++c) {
     ChainDev& ch = *S.chains[c];
-    hipLaunchKernelGGL(k_fill, dim3(grid_blocks((long)ch.nblk * g.m)), dim3(NTA), 0, s, ch.blk.p,
-                       (long)ch.nblk * g.m, 0.0);
+    hipLaunchKernelGGL(k_fill, dim3(grid_blocks((long)ch.nblk * g.ms)), dim3(NTA), 0, s, ch.blk.p,
+                       (long)ch.nblk * g.ms, 0.0);
   }
   for (int r = 0; r < P.nround; ++r) {
     const StepTask* tk = S.ck_tasks.p + (size_t)r * 2 * nc;
@@ -1018,8 +1133,8 @@ void ck_simpson_rounds(System& S, hipStream_t s) {
       a.nblk = ch.nblk;
       for (int b = 0; b <= ch.nblk; ++b) a.bnd[b] = ch.bnd[b];
       for (int b = 0; b < ch.nblk; ++b) a.ds[b] = ch.ds[b];
-      hipLaunchKernelGGL(k_simpson_seg, dim3(grid_blocks(g.m)), dim3(NTA), 0, s, ch.seg.p,
-                         ch.seg.p + (size_t)ch.segpts * g.m, g.m, a, lo, hi, hi == ch.ns ? 1 : 0,
+      hipLaunchKernelGGL(k_simpson_seg, dim3(grid_blocks(g.ms)), dim3(NTA), 0, s, ch.seg.p,
+                         ch.seg.p + (size_t)ch.segpts * g.ms, g.ms, a, lo, hi, hi == ch.ns ? 1 : 0,
                          ch.blk.p);
     }
   }
@@ -1028,6 +1143,10 @@ void ck_simpson_rounds(System& S, hipStream_t s) {
 
 void startup(System& S, double chain_step) {
   REQUIRE(S.have_chem, "set_chemistry must precede startup");
+  S.g.set_sym(S.no_sym ? 0 : S.sym_code);
+  S.sym_bad = false;
+  S.last = nullptr;
+  S.full.reset();
   const Grid& g = S.g;
   S.chains.clear();
   for (int c = 0; c < S.nchain; ++c) {
@@ -1045,7 +1164,7 @@ void startup(System& S, double chain_step) {
     for (int b = 0; b <= ch->nblk; ++b) ch->bnd[b] = bgn[b] - 1;
     ch->ns = ch->bnd[ch->nblk];
     ch->length = S.chain_length[c];
-    ch->m_ = g.m;
+    ch->m_ = g.ms;
     if (S.ck_stride > 0) {
       const int K = S.ck_stride;
       ch->slot.assign(ch->ns + 1, -1);
@@ -1054,25 +1173,26 @@ void startup(System& S, double chain_step) {
         if (sp % K == 0 || (ch->ns - sp) % K == 0) ch->slot[sp] = ch->nslot++;
       ch->dslot.upload(ch->slot.data(), ch->slot.size(), S.st.s);
       ch->segpts = std::min(K, ch->ns) + 1;
-      ch->seg.alloc((size_t)4 * ch->segpts * g.m);
-      ch->blk.alloc((size_t)ch->nblk * g.m);
+      ch->seg.alloc((size_t)4 * ch->segpts * g.ms);
+      ch->blk.alloc((size_t)ch->nblk * g.ms);
     } else {
       ch->nslot = ch->ns + 1;
     }
-    ch->qf.alloc((size_t)ch->nslot * g.m);
-    ch->qr.alloc((size_t)ch->nslot * g.m);
-    ch->fac.alloc((size_t)ch->nblk * (2 * g.m + 2 * g.mk));
+    ch->qf.alloc((size_t)ch->nslot * g.ms);
+    ch->qr.alloc((size_t)ch->nslot * g.ms);
+    ch->fac.alloc((size_t)ch->nblk * (2 * g.ms + 2 * g.mf));
     S.chains.push_back(std::move(ch));
   }
   S.chain_step = chain_step;
   const int ntask = 2 * S.nchain;
-  S.abc.alloc((size_t)3 * g.mk * std::max(ntask, 1));
-  S.q1.alloc((size_t)g.m * std::max(ntask, 1));
+  S.abc.alloc((size_t)3 * g.mc * std::max(ntask, 1));
+  S.q1.alloc((size_t)g.ms * std::max(ntask, 1));
   S.tasks.alloc(std::max(ntask, 1));
   S.omega_grid.alloc((size_t)S.nmon * g.m);
   S.rho_grid.alloc((size_t)S.nmon * g.m);
   S.part.alloc(1024);
-  S.qdev.alloc(S.nchain + S.nsolv + 1);
+  S.qdev.alloc(S.nchain + S.nsolv + 2);    // Q, a scratch value, the symmetry flag
+  hipLaunchKernelGGL(k_fill, dim3(1), dim3(NTA), 0, S.st.s, S.qdev.p, (long)S.qdev.n, 0.0);
   S.chem_dev.alloc(2 * (S.nchain + S.nsolv) + 2);
   // sweep tasks: forward (qf) and backward (qr) sweep of every chain
   std::vector<StepTask> ht(ntask);
@@ -1090,19 +1210,16 @@ void startup(System& S, double chain_step) {
       t.dir = d == 0 ? 1 : -1;
       t.init_one = 1;
       t.nblk = ch.nblk;
-      for (int b = 0; b <= ch.nblk; ++b) t.bnd[b] = ch.bnd[b];
-      for (int b = 0; b < ch.nblk; ++b) {
-        double* f = ch.fac.p + (size_t)b * (2 * g.m + 2 * g.mk);
-        t.e1[b] = f;
-        t.e2[b] = f + g.m;
-        t.k1[b] = f + 2 * g.m;
-        t.k2[b] = f + 2 * g.m + g.mk;
-      }
+      for (int b = 0; b <= MAXBLK; ++b) t.bnd[b] = ch.bnd[std::min(b, ch.nblk)];
+      t.fac = ch.fac.p;
+      t.fm = g.ms;
+      t.fk = g.mf;
+      t.sym = g.sym;
       const int ti = 2 * c + d;
-      t.A = S.abc.p + (size_t)(3 * ti) * g.mk;
-      t.B = t.A + g.mk;
-      t.C = t.B + g.mk;
-      t.q1 = S.q1.p + (size_t)ti * g.m;
+      t.A = S.abc.p + (size_t)(3 * ti) * g.mc;
+      t.B = t.A + g.mc;
+      t.C = t.B + g.mc;
+      t.q1 = S.q1.p + (size_t)ti * g.ms;
     }
   }
   if (ntask > 0)
@@ -1123,6 +1240,26 @@ void startup(System& S, double chain_step) {
 
 // ---- density() in phases, each enqueued on stream s (src/scf_mod.fp.f90:144-229)
 
+// The basis's symmetric planes hold for a cell: an operation with a s = -1
+// besides (a = -1 with z -> z + c, a = +1 with z -> -z) also has to leave |k|
+// unchanged, i.e. the third reciprocal vector normal to the other two.
+bool sym_usable(const System& S) {
+  if (!S.g.sym) return true;
+  if (S.sym_bad || S.sym_code != S.g.sym) return false;
+  if (!((S.g.sym & SYM_T) && (S.g.sym >> 2 & 1)) && !((S.g.sym & SYM_R) && !(S.g.sym >> 5 & 1))) return true;
+  auto dot = [&](int i, int j) {
+    return S.gb[i * 3] * S.gb[j * 3] + S.gb[i * 3 + 1] * S.gb[j * 3 + 1] + S.gb[i * 3 + 2] * S.gb[j * 3 + 2];
+  };
+  const double n3 = dot(2, 2);
+  return std::fabs(dot(2, 0)) <= 1e-12 * std::sqrt(n3 * dot(0, 0)) &&
+         std::fabs(dot(2, 1)) <= 1e-12 * std::sqrt(n3 * dot(1, 1));
+}
+// after the stream is synchronised: the omega of the last density_pre is not symmetric
+bool sym_failed(System& S) {
+  if (S.g.sym && S.pin_q.p[S.nchain + S.nsolv + 1] == S.sym_epoch) S.sym_bad = true;
+  return S.sym_bad;
+}
+
 // omega stars -> grid (no 1/M, :182-185), propagator factors per block
 // (make_propg), chemistry scalars for the device
 // (grid_in: S.omega_grid already holds the omega grids, star input unused;
@@ -1141,14 +1278,29 @@ void density_pre(System& S, const double* omega, const double* phi_c, const doub
     S.omega_in.alloc(nst);
     HIPCHK(hipMemcpyAsync(S.omega_in.p, S.pin_in.p, sizeof(double) * nst, hipMemcpyHostToDevice, s));
     basis_to_grid(S, S.omega_in.p, S.nmon, S.omega_grid.p, s);
+    if (g.sym) {
+      // the planes left out have to hold what the stored ones say, to rounding
+      // (against a bound of |omega|)
+      double bound = 0.0;
+      for (int a = 0; a < S.nmon; ++a) {
+        double b = 0.0;
+        for (int i = 0; i < S.nstar; ++i) b += std::fabs(omega[a + (size_t)S.nmon * i]) * S.star_bound[i];
+        bound = std::max(bound, b);
+      }
+      S.sym_epoch += 1.0;
+      hipLaunchKernelGGL(k_sym_check, dim3(grid_blocks((g.m - g.ms) * S.nmon)), dim3(NTA), 0, s,
+                         S.omega_grid.p, S.nmon, g.sym, g.n1, g.n2, g.n3, 1e-12 * bound, S.sym_epoch,
+                         S.qdev.p + S.nchain + S.nsolv + 1);
+    }
   }
   for (int c = 0; c < S.nchain; ++c) {
     ChainDev& ch = *S.chains[c];
     for (int b = 0; b < ch.nblk; ++b) {
-      double* f = ch.fac.p + (size_t)b * (2 * g.m + 2 * g.mk);
-      hipLaunchKernelGGL(k_make_propg, dim3(grid_blocks(g.m)), dim3(NTA), 0, s, ch.ds[b],
-                         S.kuhn[ch.mon[b]], S.ksq.p, g.mk, S.omega_grid.p + (size_t)ch.mon[b] * g.m,
-                         g.m, f, f + g.m, f + 2 * g.m, f + 2 * g.m + g.mk);
+      double* f = ch.fac.p + (size_t)b * (2 * g.ms + 2 * g.mf);
+      hipLaunchKernelGGL(k_make_propg, dim3(grid_blocks(std::max(g.ms, g.mf))), dim3(NTA), 0, s, ch.ds[b],
+                         S.kuhn[ch.mon[b]], S.ksq.p, g.mf, S.omega_grid.p + (size_t)ch.mon[b] * g.m,
+                         g.ms, g.n1, g.n2, g.zs->zw, (double)g.m, f, f + g.ms, f + 2 * g.ms,
+                         f + 2 * g.ms + g.mf);
     }
   }
   S.h_chem.assign(2 * (S.nchain + S.nsolv) + 2, 0.0);
@@ -1200,7 +1352,7 @@ void density_post(System& S, double* rho, hipStream_t s) {
   const Grid& g = S.g;
   for (int c = 0; c < S.nchain; ++c) {
     ChainDev& ch = *S.chains[c];
-    dev_sum(ch.point(+1, ch.ns), g.m, 1.0 / (double)g.m, S.part.p, S.qdev.p + c, s);
+    dev_sum(g, ch.point(+1, ch.ns), 1.0 / (double)g.m, S.part.p, S.qdev.p + c, s);
   }
   hipLaunchKernelGGL(k_fill, dim3(grid_blocks((long)S.nmon * g.m)), dim3(NTA), 0, s, S.rho_grid.p,
                      (long)S.nmon * g.m, 0.0);
@@ -1240,21 +1392,23 @@ void density_post(System& S, double* rho, hipStream_t s) {
     a.chain_length = ch.length;
     a.ensemble = S.chain_ens;
     if (S.ck_stride > 0)
-      hipLaunchKernelGGL(k_block_rho, dim3(grid_blocks(g.m)), dim3(NTA), 0, s, ch.blk.p, g.m, a,
-                         S.qdev.p + c, S.chem_dev.p + 2 * c, S.rho_grid.p);
+      hipLaunchKernelGGL(k_block_rho, dim3(grid_blocks(g.ms)), dim3(NTA), 0, s, ch.blk.p, g.ms, g.m, a,
+                         S.qdev.p + c, S.chem_dev.p + 2 * c, g.n1, g.n2, S.rho_grid.p);
     else
-      hipLaunchKernelGGL(k_simpson, dim3(grid_blocks(g.m)), dim3(NTA), 0, s, ch.qf.p, ch.qr.p, g.m,
-                         a, S.qdev.p + c, S.chem_dev.p + 2 * c, S.rho_grid.p);
+      hipLaunchKernelGGL(k_simpson, dim3(grid_blocks(g.ms)), dim3(NTA), 0, s, ch.qf.p, ch.qr.p, g.ms, g.m,
+                         a, S.qdev.p + c, S.chem_dev.p + 2 * c, g.n1, g.n2, S.rho_grid.p);
   }
+  if (g.sym)
+    hipLaunchKernelGGL(k_sym_expand, dim3(grid_blocks((g.m - g.ms) * S.nmon)), dim3(NTA), 0, s, S.rho_grid.p,
+                       S.nmon, g.sym, g.n1, g.n2, g.n3);
   const size_t nst = (size_t)S.nmon * S.nstar;
   if (rho) {
     S.rho_out.alloc(nst);
     grid_to_basis(S, S.rho_grid.p, S.nmon, 1.0 / (double)g.m, S.rho_out.p, s);
   }
   HIPCHK(hipGetLastError());
-  S.pin_q.alloc(S.nchain + S.nsolv);
-  HIPCHK(hipMemcpyAsync(S.pin_q.p, S.qdev.p, sizeof(double) * (S.nchain + S.nsolv),
-                        hipMemcpyDeviceToHost, s));
+  S.pin_q.alloc(S.qdev.n);
+  HIPCHK(hipMemcpyAsync(S.pin_q.p, S.qdev.p, sizeof(double) * S.qdev.n, hipMemcpyDeviceToHost, s));
   S.rho_dst = rho;
   if (rho) {
     S.pin_rho.alloc(nst);
@@ -1283,14 +1437,41 @@ void density_finish(System& S, double* qout, double* qsolv, double* phi_c, doubl
   S.have_density = true;
 }
 
+System& full_of(System& S);
+
+// density() by the system's companion that stores every plane
+template <class F>
+void on_full(System& S, F&& run) {
+  System& D = full_of(S);
+  D.profile = S.profile;
+  run(D);
+  for (int k = 0; k < 5; ++k) {
+    S.prof_ms[k] += D.prof_ms[k];
+    S.prof_n[k] += D.prof_n[k];
+    D.prof_ms[k] = 0.0;
+    D.prof_n[k] = 0;
+  }
+  S.h_Q = D.h_Q;
+  S.have_density = true;
+  ++S.density_gen;
+  S.last = &D;
+}
+
 void density(System& S, const double* omega, double* rho, double* qout, double* qsolv, double* phi_c,
              double* mu_c, double* phi_s, double* mu_s) {
-  hipStream_t s = S.st.s;
-  density_pre(S, omega, phi_c, mu_c, phi_s, mu_s, s, false, qout != nullptr);
-  density_sweeps(S, s);
-  density_post(S, rho, s);
-  S.st.sync();
-  density_finish(S, qout, qsolv, phi_c, mu_c, phi_s, mu_s);
+  if (sym_usable(S)) {
+    hipStream_t s = S.st.s;
+    density_pre(S, omega, phi_c, mu_c, phi_s, mu_s, s, false, qout != nullptr);
+    density_sweeps(S, s);
+    density_post(S, rho, s);
+    S.st.sync();
+    if (!sym_failed(S)) {
+      density_finish(S, qout, qsolv, phi_c, mu_c, phi_s, mu_s);
+      S.last = nullptr;
+      return;
+    }
+  }
+  on_full(S, [&](System& D) { density(D, omega, rho, qout, qsolv, phi_c, mu_c, phi_s, mu_s); });
 }
 
 // density() on real-space grids held in device memory: omega_grid (M, N_monomer)
@@ -1298,6 +1479,12 @@ void density(System& S, const double* omega, double* rho, double* qout, double* 
 void density_grid(System& S, const double* omega_grid, double* rho_grid, double* qout, double* qsolv,
                   double* phi_c, double* mu_c, double* phi_s, double* mu_s) {
   REQUIRE(S.started, "system not ready (startup)");
+  if (S.g.sym) {                 // grid fields need not have the basis's symmetry
+    on_full(S, [&](System& D) {
+      density_grid(D, omega_grid, rho_grid, qout, qsolv, phi_c, mu_c, phi_s, mu_s);
+    });
+    return;
+  }
   hipStream_t s = S.st.s;
   const size_t n = (size_t)S.nmon * S.g.m;
   HIPCHK(hipMemcpyAsync(S.omega_grid.p, omega_grid, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
@@ -1334,17 +1521,21 @@ struct Multi {
   }
 };
 
-System::~System() = default;
+System::~System() {
+  for (auto e : ev) (void)hipEventDestroy(e);
+  drop_graph();
+  drop_ck_graph();
+}
 
 // device bytes of one copy of S (contour storage, factors, step work)
 size_t system_bytes(const System& S) {
   const Grid& g = S.g;
   size_t b = 0;
   for (const auto& ch : S.chains) {
-    b += (size_t)2 * ch->nslot * g.m * 8 + (size_t)ch->nblk * (2 * g.m + 2 * g.mk) * 8;
-    if (S.ck_stride > 0) b += (size_t)(4 * ch->segpts + ch->nblk) * g.m * 8;
+    b += (size_t)2 * ch->nslot * g.ms * 8 + (size_t)ch->nblk * (2 * g.ms + 2 * g.mf) * 8;
+    if (S.ck_stride > 0) b += (size_t)(4 * ch->segpts + ch->nblk) * g.ms * 8;
   }
-  b += (size_t)2 * S.nchain * (3 * g.mk * 16 + g.m * 8);
+  b += (size_t)2 * S.nchain * (3 * g.mc * 16 + g.ms * 8);
   b += (size_t)(2 * S.nmon + 4) * g.m * 8 + (size_t)2 * S.nmon * g.mk * 16;
   return b;
 }
@@ -1364,6 +1555,7 @@ void copy_system(System& D, const System& S) {
   D.star_of_wave.upload(D.h_star_of_wave.data(), D.nwave, D.st.s);
   D.star_invert.upload(D.h_star_invert.data(), D.nstar, D.st.s);
   build_basis_maps(D);
+  D.sym_code = S.sym_code;
   D.have_basis = true;
   for (int i = 0; i < 9; ++i) D.gb[i] = S.gb[i];
   apply_cell(D);
@@ -1382,6 +1574,44 @@ void copy_system(System& D, const System& S) {
   D.use_graph = S.use_graph;
   startup(D, S.chain_step);
 }
+
+void set_copy_cell(System& D, const System& S) {
+  bool same = true;
+  for (int i = 0; i < 9; ++i) same = same && D.gb[i] == S.gb[i];
+  if (same) return;
+  for (int i = 0; i < 9; ++i) D.gb[i] = S.gb[i];
+  apply_cell(D);
+  D.st.sync();
+}
+
+// S's companion that stores every plane, at S's current state
+System& full_of(System& S) {
+  if (S.full && (S.full_basis != S.gen_basis || S.full_start != S.gen_start)) {
+    if (S.last) S.have_density = false;
+    S.last = nullptr;
+    S.full.reset();
+  }
+  if (!S.full) {
+    auto D = std::make_unique<System>();
+    D->no_sym = true;
+    copy_system(*D, S);
+    S.full_basis = S.gen_basis;
+    S.full_start = S.gen_start;
+    S.full = std::move(D);
+  }
+  System& D = *S.full;
+  set_copy_cell(D, S);
+  if (D.use_graph != S.use_graph) {
+    D.use_graph = S.use_graph;
+    D.drop_graph();
+    D.drop_ck_graph();
+  }
+  D.chi = S.chi;
+  return D;
+}
+
+// the system that holds the results of S's last density()
+System& live(System& S) { return S.last ? *S.last : S; }
 
 // at least P copies matching S's current state (cell refreshed on every call)
 void ensure_multi(System& S, int P) {
@@ -1407,17 +1637,12 @@ void ensure_multi(System& S, int P) {
     S.multi = std::move(M);
   }
   for (auto& D : S.multi->cl) {
-    bool same = true;
-    for (int i = 0; i < 9; ++i) same = same && D->gb[i] == S.gb[i];
-    if (!same) {
-      for (int i = 0; i < 9; ++i) D->gb[i] = S.gb[i];
-      apply_cell(*D);
-      D->st.sync();
-    }
+    set_copy_cell(*D, S);
     D->use_graph = S.use_graph;
   }
 }
 
+void stress(System& S, int ncp, const double* dgsq, const double* phi_c, const double* mu_c, double* out);
 void stress_launch(System& S, int ncp, const double* dgsq, hipStream_t s);
 void stress_finish(System& S, int ncp, const double* phi_c, const double* mu_c, double* out);
 
@@ -1498,6 +1723,18 @@ void density_many(System& S, int n, const double* omega, double* rho, double* qo
       }
     S.st.sync();
     for (int i = 0; i < cnt; ++i) {
+      System& D = *Mu.cl[i];
+      if (!sym_usable(D) || sym_failed(D)) {     // this field or cell needs every plane
+        density(D, omega + (size_t)(k0 + i) * nst, rho + (size_t)(k0 + i) * nst,
+                qout ? qout + (size_t)(k0 + i) * S.nchain : nullptr,
+                qsolv ? qsolv + (size_t)(k0 + i) * S.nsolv : nullptr, phi_c, mu_c, phi_s, mu_s);
+        if (stress_out)
+          stress(live(D), ncp, dgsq + (size_t)(k0 + i) * S.nstar * ncp, phi_c, mu_c,
+                 stress_out + (size_t)(k0 + i) * ncp);
+        D.sym_bad = false;                       // another field may be symmetric
+        continue;
+      }
+      D.last = nullptr;
       density_finish(*Mu.cl[i], qout ? qout + (size_t)(k0 + i) * S.nchain : nullptr,
                      qsolv ? qsolv + (size_t)(k0 + i) * S.nsolv : nullptr, phi_c, mu_c, phi_s, mu_s);
       if (stress_out) stress_finish(*Mu.cl[i], ncp, phi_c, mu_c, stress_out + (size_t)(k0 + i) * ncp);
@@ -1545,7 +1782,7 @@ void adjoint_setup(System& S, bool with_k) {
     A->keepk.alloc((size_t)3 * g.mk * A->ntask);
     A->kblk.alloc((size_t)g.mk * nblk);
   }
-  A->abc.alloc((size_t)3 * g.mk * A->ntask);
+  A->abc.alloc((size_t)3 * g.mc * A->ntask);
   A->q1.alloc((size_t)g.m * A->ntask);
   A->gblk.alloc((size_t)g.m * nblk);
   A->tasks.alloc(A->ntask);
@@ -1583,9 +1820,9 @@ void adjoint_setup(System& S, bool with_k) {
         t.add_src = 0;
         t.rev = t.reload = t.nostore = 1;
       }
-      t.A = A->abc.p + (size_t)(3 * ti) * g.mk;
-      t.B = t.A + g.mk;
-      t.C = t.B + g.mk;
+      t.A = A->abc.p + (size_t)(3 * ti) * g.mc;
+      t.B = t.A + g.mc;
+      t.C = t.B + g.mc;
       t.q1 = A->q1.p + (size_t)ti * g.m;
       t.keepU = A->keep.p + (size_t)(5 * ti) * g.m;
       t.keepV = t.keepU + g.m;
@@ -1611,7 +1848,7 @@ void adjoint_setup(System& S, bool with_k) {
     // segment buffers of a chain: 0 q_f(R_r), 1 q_r(R_r), 2 q_f(F_r), 3 q_r(F_r)
     const int K = S.ck_stride, nc = S.nchain;
     const CkPlan& P = S.ck;
-    A->rec_abc.alloc((size_t)3 * g.mk * 4 * nc);
+    A->rec_abc.alloc((size_t)3 * g.mc * 4 * nc);
     A->rec_q1.alloc((size_t)g.m * 4 * nc);
     std::vector<StepTask> rec((size_t)P.nround * 4 * nc), adj((size_t)P.nround * 4 * nc);
     for (int r = 0; r < P.nround; ++r)
@@ -1644,9 +1881,9 @@ void adjoint_setup(System& S, bool with_k) {
           t.slab = seg(2 * side + d);
           t.pmap = side == 0 ? mapR : mapF;
           const int ti = 4 * c + k;
-          t.A = A->rec_abc.p + (size_t)(3 * ti) * g.mk;
-          t.B = t.A + g.mk;
-          t.C = t.B + g.mk;
+          t.A = A->rec_abc.p + (size_t)(3 * ti) * g.mc;
+          t.B = t.A + g.mc;
+          t.C = t.B + g.mc;
           t.q1 = A->rec_q1.p + (size_t)ti * g.m;
           if (lo >= hi) {
             t.skip = 1;
@@ -1703,16 +1940,16 @@ void run_adj_sweeps(const Grid& g, const AdjSweeps& W, hipStream_t s) {
         run_sweeps(g, W.ck_rec + (size_t)r * nt, nt, W.len[r], s);
       tasks = W.ck_adj + (size_t)r * nt;
     }
-    launch_step_a(g, tasks, nt, j, s);
+    launch_step_a(g, tasks, nt, j, true, s);
     if (j >= 1)
       hipLaunchKernelGGL(k_adj_grad, dim3(gb), dim3(256), 0, s, tasks, W.pairs, W.npair, j - 1, g.m);
     if (j == max_ns) break;
-    g.step_z(tasks, nt, j, 0, 2, s);
-    g.step_c(tasks, nt, j, s);
-    g.step_z(tasks, nt, j, 1, 1, s);
+    g.step_z(tasks, nt, j, 0, 2, true, s);
+    g.step_c(tasks, nt, j, true, s);
+    g.step_z(tasks, nt, j, 1, 1, true, s);
     if (W.with_k)
       hipLaunchKernelGGL(k_adj_kgrad, dim3(gk), dim3(256), 0, s, tasks, W.pairs, W.npair, j, g.n1,
-                         g.mk, (double)g.m);
+                         g.n2, g.n3, g.zs->zw);
   }
   HIPCHK(hipGetLastError());
 }
@@ -1771,6 +2008,10 @@ void adjoint_pre(System& S, const double* lam, const double* dQ, bool with_k, Ad
   const Grid& g = S.g;
   hipStream_t s = S.st.s;
   const int nb = ADJ_NB;
+  // lam in the sweeps' packed order
+  hipLaunchKernelGGL(k_pack, dim3(grid_blocks(S.nmon * g.m)), dim3(NTA), 0, s, lam, g.m, S.nmon, g.n1, g.n2,
+                     A.lam.p);
+  lam = A.lam.p;
   double* part = A.part.p;
   auto& T = C.T;
   auto& coef = C.coef;
@@ -1809,8 +2050,7 @@ void adjoint_pre(System& S, const double* lam, const double* dQ, bool with_k, Ad
     for (int b = 0; b < ch.nblk; ++b) tsum += T[c][b];
     gam[c] = (dQ ? dQ[c] : 0.0) - (S.chain_ens == 1 ? 0.0 : coef[c] * tsum / Q);
   }
-  // sources: lam copied into the adjoint state, coefficient and end term per chain
-  HIPCHK(hipMemcpyAsync(A.lam.p, lam, sizeof(double) * S.nmon * g.m, hipMemcpyDeviceToDevice, s));
+  // sources: coefficient and end term per chain
   std::vector<double> hs(2 * S.nchain);
   for (int c = 0; c < S.nchain; ++c) {
     hs[2 * c] = coef[c];
@@ -1845,7 +2085,8 @@ void adjoint_post(System& S, const AdjCall& C, double* grad, int ncp, const doub
     ChainDev& ch = *S.chains[c];
     for (int b = 0; b < ch.nblk; ++b)
       hipLaunchKernelGGL(k_axpy1, dim3(grid_blocks(g.m)), dim3(NTA), 0, s,
-                         A.gblk.p + (A.blk_off[c] + b) * g.m, g.m, grad + (size_t)ch.mon[b] * g.m);
+                         A.gblk.p + (A.blk_off[c] + b) * g.m, g.m, g.n1, g.n2,
+                         grad + (size_t)ch.mon[b] * g.m);
   }
   HIPCHK(hipGetLastError());
   GeomArgs ga;
@@ -1887,8 +2128,10 @@ void adjoint_post(System& S, const AdjCall& C, double* grad, int ncp, const doub
       for (int b = 0; b < ch.nblk; ++b) tsum += T[c][b];
       for (int b = 0; b < ch.nblk; ++b, ++o) {
         const double* gb_ = A.gblk.p + (A.blk_off[c] + b) * g.m;
-        hipLaunchKernelGGL(k_partial_dot, dim3(nb), dim3(NTA), 0, s, gb_,
-                           S.omega_grid.p + (size_t)ch.mon[b] * g.m, g.m, part);
+        // omega in packed order, into a buffer that is free after the sweeps
+        hipLaunchKernelGGL(k_pack, dim3(grid_blocks(g.m)), dim3(NTA), 0, s,
+                           S.omega_grid.p + (size_t)ch.mon[b] * g.m, g.m, 1, g.n1, g.n2, A.keep.p);
+        hipLaunchKernelGGL(k_partial_dot, dim3(nb), dim3(NTA), 0, s, gb_, A.keep.p, g.m, part);
         const double t1 = host_sum(S, part, nb);
         hipLaunchKernelGGL(k_partial_dot, dim3(nb), dim3(NTA), 0, s, A.kblk.p + (A.blk_off[c] + b) * g.mk,
                            S.ksq.p, g.mk, part);
@@ -1902,8 +2145,47 @@ void adjoint_post(System& S, const AdjCall& C, double* grad, int ncp, const doub
   S.st.sync();
 }
 
-void density_adjoint(System& S, const double* lam, const double* dQ, double* grad, int ncp,
+// The system whose stored planes the reverse mode of S's last density() reads:
+// every plane, since adjoint fields need not be symmetric.  After a density()
+// on symmetric planes the companion takes over its fields and contour points.
+System& adjoint_of(System& S) {
+  REQUIRE(S.have_density, "the adjoint requires a previous density()");
+  System& L = live(S);
+  if (!L.g.sym) return L;
+  System& D = full_of(S);
+  const Grid& g = S.g;
+  hipStream_t s = D.st.s;
+  S.st.sync();
+  const size_t n = sizeof(double) * (size_t)S.nmon * g.m;
+  HIPCHK(hipMemcpyAsync(D.omega_grid.p, S.omega_grid.p, n, hipMemcpyDeviceToDevice, s));
+  HIPCHK(hipMemcpyAsync(D.rho_grid.p, S.rho_grid.p, n, hipMemcpyDeviceToDevice, s));
+  const double* hc = S.h_chem.data();
+  std::vector<double> phi(S.nchain), mu(S.nchain), phis(S.nsolv), mus(S.nsolv);
+  for (int c = 0; c < S.nchain; ++c) phi[c] = hc[2 * c], mu[c] = hc[2 * c + 1];
+  for (int i = 0; i < S.nsolv; ++i) phis[i] = hc[2 * (S.nchain + i)], mus[i] = hc[2 * (S.nchain + i) + 1];
+  density_pre(D, nullptr, phi.data(), mu.data(), phis.data(), mus.data(), s, true, S.chain_ens == 1);
+  for (int c = 0; c < S.nchain; ++c) {
+    ChainDev &a = *S.chains[c], &b = *D.chains[c];
+    const auto expand = [&](const double* from, double* to, int np) {
+      hipLaunchKernelGGL(k_sym_point, dim3(grid_blocks(g.m), np), dim3(NTA), 0, s, from, g.ms, g.sym, g.n1,
+                         g.n2, g.n3, 1, to, g.m);
+    };
+    expand(a.qf.p, b.qf.p, a.nslot);
+    expand(a.qr.p, b.qr.p, a.nslot);
+    if (S.ck_stride > 0) expand(a.blk.p, b.blk.p, a.nblk);
+  }
+  HIPCHK(hipGetLastError());
+  D.st.sync();
+  D.h_Q = S.h_Q;
+  D.chain_ens = S.chain_ens;
+  D.have_density = true;
+  S.last = &D;
+  return D;
+}
+
+void density_adjoint(System& sys, const double* lam, const double* dQ, double* grad, int ncp,
                      const double* dgg, double* dcell, double* dlen, double* dphi) {
+  System& S = adjoint_of(sys);
   REQUIRE(ncp <= 6, "at most 6 cell parameters");
   const bool with_k = dgg != nullptr || dlen != nullptr;
   AdjCall C;
@@ -1934,7 +2216,8 @@ void density_adjoint(System& S, const double* lam, const double* dQ, double* gra
 // every system's tasks run the kernels of its lone adjoint, so the results
 // equal the single calls'.
 struct AdjGroup {
-  std::vector<System*> sys;
+  std::vector<System*> members;  // as given
+  std::vector<System*> sys;      // those whose planes their adjoints read (adjoint_of)
   std::vector<uint64_t> ids;     // AdjState ids the launch set was built from
   bool with_k = false;
   Stream st;
@@ -2022,7 +2305,7 @@ void build_adj_group(AdjGroup& G) {
 void adjoint_group(AdjGroup& G, const double* const* lam, const double* const* dQ,
                    double* const* grad, const int* ncp, const double* const* dgg,
                    double* const* dcell, double* const* dlen, double* const* dphi) {
-  const size_t n = G.sys.size();
+  const size_t n = G.members.size();
   bool with_k = false;
   for (size_t i = 0; i < n; ++i) {
     REQUIRE(lam && lam[i] && grad && grad[i], "null grid pointer");
@@ -2031,6 +2314,8 @@ void adjoint_group(AdjGroup& G, const double* const* lam, const double* const* d
     REQUIRE(!(dgg && dgg[i]) || (dcell && dcell[i]), "dGG given without an output for the cell gradient");
     with_k = with_k || (dgg && dgg[i]) || (dlen && dlen[i]);
   }
+  G.sys.clear();
+  for (System* S : G.members) G.sys.push_back(&adjoint_of(*S));
   std::vector<AdjCall> C(n);
   for (size_t i = 0; i < n; ++i)
     adjoint_pre(*G.sys[i], lam[i], dQ ? dQ[i] : nullptr, with_k, C[i]);
@@ -2073,9 +2358,10 @@ void stress_launch(System& S, int ncp, const double* dgsq, hipStream_t s) {
   HIPCHK(hipMemcpyAsync(S.dgsq.p, S.pin_dgsq.p, sizeof(double) * S.nstar * ncp,
                         hipMemcpyHostToDevice, s));
   const int chunk = 32;
-  const long mkc = (long)g.n3 * S.ncolp;      // one point's compact spectrum
+  const long mkc = (long)g.n3 * S.ncol;       // one point's compact spectrum
   S.sbasis.alloc((size_t)2 * chunk * S.nstar);
-  S.skbuf.alloc((size_t)2 * chunk * mkc);
+  S.skbuf.alloc((size_t)2 * chunk * (mkc + (long)g.np * S.nin));
+  double2* const work = S.skbuf.p + (size_t)2 * chunk * mkc;
   size_t npts = 0;
   for (int sp = 0; sp < S.nchain; ++sp) npts += (size_t)S.chains[sp]->ns + 1;
   S.sdots.alloc(npts * ncp);
@@ -2086,8 +2372,8 @@ void stress_launch(System& S, int ncp, const double* dgsq, hipStream_t s) {
       const int np = std::min(chunk, ch.ns + 1 - p0);
       // qf and qr of the chunk's points in one launch per pass: qr's spectra
       // after qf's, then star coefficients (2 np, N_star) with qr's at np + p
-      g.r2c_cols(ch.qf.p + (size_t)p0 * g.m, ch.qr.p + (size_t)p0 * g.m, S.skbuf.p, np, S.scpos.p,
-                 S.ncol, S.ncolp, s);
+      g.r2c_cols(ch.qf.p + (size_t)p0 * g.ms, ch.qr.p + (size_t)p0 * g.ms, work, S.skbuf.p, np, S.scpos.p,
+                 S.nin, S.ncol, S.ssrc.p, S.scolk.p, s);
       hipLaunchKernelGGL(k_kgrid_to_basis, dim3(grid_blocks((long)S.nstar * 2 * np)), dim3(NTA), 0,
                          s, S.skbuf.p, mkc, 2 * np, S.nstar, S.sidx_c.p, S.sconj.p, S.scoef.p,
                          S.star_invert.p, 1.0, S.sbasis.p, 0);
@@ -2189,7 +2475,7 @@ struct BatchInst {
 };
 
 struct Group {
-  int n1 = 0, n2 = 0, n3 = 0;
+  int n1 = 0, n2 = 0, n3 = 0, np = 0;
   std::vector<int> members;
   // the members' chain-discretisation generations when the tasks were
   // copied: a restart (startup, set_checkpoint) frees the slabs the tasks
@@ -2239,13 +2525,14 @@ void build_groups(Batch& Bt) {
     System& S = *Bt.inst[i].S;
     Group* G = nullptr;
     for (auto& g : Bt.groups)
-      if (g->n1 == S.g.n1 && g->n2 == S.g.n2 && g->n3 == S.g.n3) G = g.get();
+      if (g->n1 == S.g.n1 && g->n2 == S.g.n2 && g->n3 == S.g.n3 && g->np == S.g.np) G = g.get();
     if (!G) {
       Bt.groups.push_back(std::make_unique<Group>());
       G = Bt.groups.back().get();
       G->n1 = S.g.n1;
       G->n2 = S.g.n2;
       G->n3 = S.g.n3;
+      G->np = S.g.np;
     }
     G->members.push_back(i);
     G->gen_start.push_back(S.gen_start);
@@ -2293,6 +2580,14 @@ void batch_density(Batch& Bt, bool with_stress) {
   for (auto& B : Bt.inst) {
     if (!B.active) continue;
     System& S = *B.S;
+    if (!sym_usable(S) || sym_failed(S)) {       // this field or cell needs every plane
+      density(S, B.omega.data(), B.rho.data(), B.q.data(), B.qs.data(), B.phi_c.data(), B.mu_c.data(),
+              B.phi_s.data(), B.mu_s.data());
+      if (with_stress)
+        stress(live(S), B.ncp, B.dgsq.data(), B.phi_c.data(), B.mu_c.data(), B.stress.data());
+      continue;
+    }
+    S.last = nullptr;
     density_finish(S, B.q.data(), B.qs.data(), B.phi_c.data(), B.mu_c.data(), B.phi_s.data(),
                    B.mu_s.data());
     if (with_stress) stress_finish(S, B.ncp, B.phi_c.data(), B.mu_c.data(), B.stress.data());
@@ -2442,9 +2737,7 @@ void batch_solve(Batch& Bt) {
   // fixed cell: residual stress of the final fields (:1473)
   if (!Bt.domain) {
     for (auto& B : Bt.inst) {
-      stress_launch(*B.S, B.ncp, B.dgsq.data(), B.S->st.s);
-      B.S->st.sync();
-      stress_finish(*B.S, B.ncp, B.phi_c.data(), B.mu_c.data(), B.stress.data());
+      stress(live(*B.S), B.ncp, B.dgsq.data(), B.phi_c.data(), B.mu_c.data(), B.stress.data());
     }
   }
 }
@@ -2561,10 +2854,10 @@ int pscf_step_create(const int ngrid[3], int64_t* step) {
       int dim = ngrid[2] > 1 ? 3 : (ngrid[1] > 1 ? 2 : 1);
       p->g.init(ngrid, dim);
       const Grid& g = p->g;
-      p->fac.alloc(2 * g.m + 2 * g.mk);
+      p->fac.alloc(2 * g.m + 2 * g.mf);
       p->slab.alloc(2 * g.m);
       p->q1.alloc(g.m);
-      p->abc.alloc(3 * g.mk);
+      p->abc.alloc(3 * g.mc);
       p->task.alloc(1);
     } catch (...) {
       delete p;
@@ -2586,7 +2879,7 @@ int pscf_step_make_propg(int64_t step, double ds, double b, const double* ksq, c
     S.om.upload(omega, g.m, S.st.s);
     double* f = S.fac.p;
     hipLaunchKernelGGL(k_make_propg, dim3(grid_blocks(g.m)), dim3(NTA), 0, S.st.s, ds, b, S.ksq.p,
-                       g.mk, S.om.p, g.m, f, f + g.m, f + 2 * g.m, f + 2 * g.m + g.mk);
+                       g.mf, S.om.p, g.m, g.n1, g.n2, g.zs->zw, (double)g.m, f, f + g.m, f + 2 * g.m, f + 2 * g.m + g.mf);
     HIPCHK(hipGetLastError());
     S.st.sync();
     S.have_propg = true;
@@ -2598,7 +2891,10 @@ int pscf_step_exp(int64_t step, const double* q_in, double* q_out) {
     StepState& S = *from_handle<StepState>(step, "step");
     REQUIRE(S.have_propg, "step_exp requires make_propg");
     const Grid& g = S.g;
-    HIPCHK(hipMemcpyAsync(S.slab.p, q_in, sizeof(double) * g.m, hipMemcpyHostToDevice, S.st.s));
+    // q1 holds the grid-order input, then output, while no kernel uses it
+    HIPCHK(hipMemcpyAsync(S.q1.p, q_in, sizeof(double) * g.m, hipMemcpyHostToDevice, S.st.s));
+    hipLaunchKernelGGL(k_pack, dim3(grid_blocks(g.m)), dim3(NTA), 0, S.st.s, S.q1.p, g.m, 1, g.n1, g.n2,
+                       S.slab.p);
     StepTask t;
     std::memset(&t, 0, sizeof t);
     t.slab = S.slab.p;
@@ -2606,22 +2902,16 @@ int pscf_step_exp(int64_t step, const double* q_in, double* q_out) {
     t.jend = 1;
     t.dir = 1;
     t.init_one = 0;
-    t.nblk = 1;
-    t.bnd[0] = 0;
-    t.bnd[1] = 1;
-    double* f = S.fac.p;
-    t.e1[0] = f;
-    t.e2[0] = f + g.m;
-    t.k1[0] = f + 2 * g.m;
-    t.k2[0] = f + 2 * g.m + g.mk;
+    one_step_blocks(t, g, S.fac.p);
     t.A = S.abc.p;
-    t.B = S.abc.p + g.mk;
-    t.C = S.abc.p + 2 * g.mk;
+    t.B = S.abc.p + g.mc;
+    t.C = S.abc.p + 2 * g.mc;
     t.q1 = S.q1.p;
     HIPCHK(hipMemcpyAsync(S.task.p, &t, sizeof t, hipMemcpyHostToDevice, S.st.s));
     run_sweeps(g, S.task.p, 1, 1, S.st.s);
-    HIPCHK(hipMemcpyAsync(q_out, S.slab.p + g.m, sizeof(double) * g.m, hipMemcpyDeviceToHost,
-                          S.st.s));
+    hipLaunchKernelGGL(k_unpack, dim3(grid_blocks(g.m)), dim3(NTA), 0, S.st.s, S.slab.p + g.m, g.m, 1,
+                       g.n1, g.n2, S.q1.p);
+    HIPCHK(hipMemcpyAsync(q_out, S.q1.p, sizeof(double) * g.m, hipMemcpyDeviceToHost, S.st.s));
     S.st.sync();
   });
 }
@@ -2639,10 +2929,10 @@ int pscf_step_exp_noalloc(const int ngrid[3], double ds, double b, const double*
     // scratch layout in doubles, every part 256-byte aligned
     const auto up = [](size_t n) { return (n + 31) / 32 * 32; };
     const size_t o_tw = up((sizeof(StepTask) + sizeof(double) - 1) / sizeof(double));
-    const size_t ntw = (size_t)g.n1 + g.n2 + g.n3;
+    const size_t ntw = (size_t)g.n1 + g.n2 + g.n3 + g.nl;
     const size_t o_fac = o_tw + up(2 * ntw);
-    const size_t o_abc = o_fac + up(2 * g.m + 2 * g.mk);
-    const size_t o_q1 = o_abc + up(6 * g.mk);
+    const size_t o_abc = o_fac + up(2 * g.m + 2 * g.mf);
+    const size_t o_q1 = o_abc + up(6 * g.mc);
     const size_t o_slab = o_q1 + up(g.m);
     const size_t need = o_slab + up(2 * g.m);
     char msg[200];
@@ -2652,43 +2942,41 @@ int pscf_step_exp_noalloc(const int ngrid[3], double ds, double b, const double*
     REQUIRE(need <= kScratchDoubles, msg);
     double* base = scratch_on_current_device();
     hipStream_t s = nullptr;                      // the default stream
-    // twiddle tables of the three edges
+    // twiddle tables of the three edges and the packed rows
     std::vector<double2> htw(ntw);
     host_twiddles(g.n1, htw.data());
     host_twiddles(g.n2, htw.data() + g.n1);
     host_twiddles(g.n3, htw.data() + g.n1 + g.n2);
+    host_twiddles(g.nl, htw.data() + g.n1 + g.n2 + g.n3);
     double2* dtw = reinterpret_cast<double2*>(base + o_tw);
     HIPCHK(hipMemcpyAsync(dtw, htw.data(), sizeof(double2) * ntw, hipMemcpyHostToDevice, s));
     g.tw1 = dtw;
     g.tw2 = dtw + g.n1;
     g.tw3 = dtw + g.n1 + g.n2;
+    g.twl = g.tw3 + g.n3;
     // make_propg (src/step_mod.f90:109-129)
     double* f = base + o_fac;
-    hipLaunchKernelGGL(k_make_propg, dim3(grid_blocks(g.m)), dim3(NTA), 0, s, ds, b, ksq, g.mk, omega,
-                       g.m, f, f + g.m, f + 2 * g.m, f + 2 * g.m + g.mk);
-    // one step (src/step_mod.f90:146-176): q_in is the start of a one-step sweep
+    hipLaunchKernelGGL(k_make_propg, dim3(grid_blocks(g.m)), dim3(NTA), 0, s, ds, b, ksq, g.mf, omega,
+                       g.m, g.n1, g.n2, g.zs->zw, (double)g.m, f, f + g.m, f + 2 * g.m, f + 2 * g.m + g.mf);
+    // one step (src/step_mod.f90:146-176): a one-step sweep from q_in
     StepTask t;
     std::memset(&t, 0, sizeof t);
     t.slab = base + o_slab;
-    t.start = q_in;
+    hipLaunchKernelGGL(k_pack, dim3(grid_blocks(g.m)), dim3(NTA), 0, s, q_in, g.m, 1, g.n1, g.n2, t.slab);
     t.ns = 1;
     t.jend = 1;
     t.dir = 1;
-    t.nblk = 1;
-    t.bnd[0] = 0;
-    t.bnd[1] = 1;
-    t.e1[0] = f;
-    t.e2[0] = f + g.m;
-    t.k1[0] = f + 2 * g.m;
-    t.k2[0] = f + 2 * g.m + g.mk;
+    one_step_blocks(t, g, f);
     t.A = reinterpret_cast<double2*>(base + o_abc);
-    t.B = t.A + g.mk;
-    t.C = t.B + g.mk;
+    t.B = t.A + g.mc;
+    t.C = t.B + g.mc;
     t.q1 = base + o_q1;
     StepTask* dtask = reinterpret_cast<StepTask*>(base);
     HIPCHK(hipMemcpyAsync(dtask, &t, sizeof t, hipMemcpyHostToDevice, s));
     run_sweeps(g, dtask, 1, 1, s);
-    HIPCHK(hipMemcpyAsync(q_out, t.slab + g.m, sizeof(double) * g.m, hipMemcpyDeviceToDevice, s));
+    hipLaunchKernelGGL(k_unpack, dim3(grid_blocks(g.m)), dim3(NTA), 0, s, t.slab + g.m, g.m, 1, g.n1, g.n2,
+                       q_out);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s));
   });
 }
@@ -2710,9 +2998,6 @@ int pscf_system_create(const int ngrid[3], int dim, int64_t* sys) {
 int pscf_system_destroy(int64_t sys) {
   return guarded([&] {
     System* S = from_handle<System>(sys, "system");
-    for (auto e : S->ev) (void)hipEventDestroy(e);
-    S->drop_graph();
-    S->drop_ck_graph();
     delete S;
   });
 }
@@ -2728,11 +3013,11 @@ int pscf_profile_step_kernel(int64_t sys, int kind, int j, int reps, double* us)
     ensure_events(S, 2);
     auto launch = [&] {
       if (kind == 0)
-        launch_step_a(g, S.tasks.p, S.ntask, j, s);
+        launch_step_a(g, S.tasks.p, S.ntask, j, false, s);
       else if (kind == 2)
-        g.step_c(S.tasks.p, S.ntask, j, s);
+        g.step_c(S.tasks.p, S.ntask, j, false, s);
       else
-        g.step_z(S.tasks.p, S.ntask, j, kind == 1 ? 0 : 1, kind == 1 ? 2 : 1, s);
+        g.step_z(S.tasks.p, S.ntask, j, kind == 1 ? 0 : 1, kind == 1 ? 2 : 1, false, s);
     };
     launch();
     HIPCHK(hipEventRecord(S.ev[0], s));
@@ -2810,6 +3095,8 @@ int pscf_system_set_basis(int64_t sys, int n_wave, int n_star, const int* wave, 
     S.star_of_wave.upload(star_of_wave, n_wave, S.st.s);
     S.star_invert.upload(star_invert, n_star, S.st.s);
     build_basis_maps(S);
+    S.sym_code = detect_sym(S);
+    S.sym_bad = false;
     S.have_basis = true;
     ++S.gen_basis;
     if (S.have_cell) {
@@ -2830,6 +3117,7 @@ int pscf_system_set_cell(int64_t sys, const double* G_basis) {
       for (int jj = 0; jj < dim; ++jj) S.gb[i * 3 + jj] = G_basis[i + dim * jj];
     apply_cell(S);
     S.st.sync();
+    S.sym_bad = false;
   });
 }
 
@@ -2889,6 +3177,10 @@ int pscf_system_set_chain_length(int64_t sys, const double* chain_length) {
       REQUIRE(chain_length[c] > 0.0, "chain length must be positive");
       S.chain_length[c] = chain_length[c];
       if (c < (int)S.chains.size()) S.chains[c]->length = chain_length[c];
+      if (S.full && c < (int)S.full->chains.size()) {
+        S.full->chain_length[c] = chain_length[c];
+        S.full->chains[c]->length = chain_length[c];
+      }
     }
   });
 }
@@ -3054,8 +3346,8 @@ int pscf_adjoint_group_create(int n, const int64_t* systems, int64_t* group) {
     auto G = std::make_unique<AdjGroup>();
     for (int i = 0; i < n; ++i) {
       System* S = from_handle<System>(systems[i], "system");
-      for (System* o : G->sys) REQUIRE(o != S, "adjoint group: a system appears twice");
-      G->sys.push_back(S);
+      for (System* o : G->members) REQUIRE(o != S, "adjoint group: a system appears twice");
+      G->members.push_back(S);
     }
     *group = reinterpret_cast<int64_t>(G.release());
   });
@@ -3099,13 +3391,13 @@ int pscf_grid_to_basis_dev(int64_t sys, const double* grid, int nf, double scale
 int pscf_scf_stress(int64_t sys, int ncp, const double* dGsq, const double* phi_chain,
                     const double* mu_chain, double* out) {
   return guarded([&] {
-    stress(*from_handle<System>(sys, "system"), ncp, dGsq, phi_chain, mu_chain, out);
+    stress(live(*from_handle<System>(sys, "system")), ncp, dGsq, phi_chain, mu_chain, out);
   });
 }
 
 int pscf_divide_energy_terms(int64_t sys, double* out) {
   return guarded([&] {
-    System& S = *from_handle<System>(sys, "system");
+    System& S = live(*from_handle<System>(sys, "system"));
     REQUIRE(S.have_density, "divide_energy requires a previous density()");
     REQUIRE(S.ck_stride == 0, "divide_energy needs every contour point (checkpointed storage is on)");
     const Grid& g = S.g;
@@ -3115,8 +3407,9 @@ int pscf_divide_energy_terms(int64_t sys, double* out) {
       for (int w = 0; w < 2; ++w) {
         const int pt = w == 0 ? nh : nt;
         const int nb = 512;
-        hipLaunchKernelGGL(k_partial_qlogq, dim3(nb), dim3(NTA), 0, S.st.s, ch.qf.p + (size_t)pt * g.m,
-                           ch.qr.p + (size_t)pt * g.m, w == 0 ? 1 : 0, g.m, S.part.p);
+        hipLaunchKernelGGL(k_partial_qlogq, dim3(nb), dim3(NTA), 0, S.st.s, ch.qf.p + (size_t)pt * g.ms,
+                           ch.qr.p + (size_t)pt * g.ms, w == 0 ? 1 : 0, g.ms, g.sym, g.n3,
+                           (long)g.n1 * g.n2, S.part.p);
         hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(NTA), 0, S.st.s, S.part.p, nb,
                            1.0 / (S.h_Q[c] * (double)g.m), S.qdev.p + S.nchain + S.nsolv);
         double v = 0.0;
@@ -3131,7 +3424,7 @@ int pscf_divide_energy_terms(int64_t sys, double* out) {
 
 int pscf_system_get_grids(int64_t sys, double* omega_grid, double* rho_grid) {
   return guarded([&] {
-    System& S = *from_handle<System>(sys, "system");
+    System& S = live(*from_handle<System>(sys, "system"));
     REQUIRE(S.have_density, "no density computed yet");
     const size_t n = (size_t)S.nmon * S.g.m;
     if (omega_grid) HIPCHK(hipMemcpy(omega_grid, S.omega_grid.p, sizeof(double) * n, hipMemcpyDeviceToHost));
@@ -3148,14 +3441,19 @@ int pscf_system_density_generation(int64_t sys, int64_t* gen) {
 
 int pscf_system_get_q(int64_t sys, int chain, int dir, int s, double* q) {
   return guarded([&] {
-    System& S = *from_handle<System>(sys, "system");
+    System& S = live(*from_handle<System>(sys, "system"));
     REQUIRE(S.have_density, "no density computed yet");
     REQUIRE(chain >= 0 && chain < S.nchain, "chain index out of range");
     ChainDev& ch = *S.chains[chain];
     REQUIRE(s >= 0 && s <= ch.ns, "contour index out of range");
     REQUIRE(S.ck_stride == 0 || ch.slot[s] >= 0, "contour point not stored (checkpointed storage)");
     const double* src = ch.point(dir > 0 ? 1 : -1, s);
-    HIPCHK(hipMemcpy(q, src, sizeof(double) * S.g.m, hipMemcpyDeviceToHost));
+    DevBuf<double> grid;
+    grid.alloc(S.g.m);
+    hipLaunchKernelGGL(k_sym_point, dim3(grid_blocks(S.g.m)), dim3(NTA), 0, S.st.s, src, 0L, S.g.sym, S.g.n1,
+                       S.g.n2, S.g.n3, 0, grid.p, 0L);
+    HIPCHK(hipMemcpyAsync(q, grid.p, sizeof(double) * S.g.m, hipMemcpyDeviceToHost, S.st.s));
+    S.st.sync();
   });
 }
 
