@@ -310,6 +310,39 @@ __host__ __device__ __forceinline__ long unpack_kindex(long i, int n1, int n2, i
   return s.kx + (n1 / 2 + 1) * (s.l + h * nl + n2 * (row / tiles));
 }
 
+// ... and back, for one plane (N3 = 1): the place of the factor of column kx
+// (any kx < N1) at ky = l + h NL.  |k| of k and -k are one, so a column kx >
+// N1/2 takes the factor of (-kx, -ky), and of the columns kx = 0 and N1/2 one
+// of l and -l is held.
+__host__ __device__ __forceinline__ int z_factor_at(int kx, int l, int h, int n1, int nl, int zw) {
+  const int kp = zw / 2, ntx = (n1 / 2 + kp - 1) / kp, nlp = nl > 1 ? nl / 2 : 1;
+  const bool edge = kx == 0 || 2 * kx == n1;
+  if (edge ? 2 * l > nl : 2 * kx > n1) {           // -> (-kx, -ky)
+    kx = edge ? kx : n1 - kx;
+    if (l) {
+      l = nl - l;
+      h = 1 - h;
+    }
+  }
+  int lp = 0, sg = 0, p = kx;
+  if (nl > 1) {
+    if (l == 0 || 2 * l == nl) {
+      sg = l != 0;
+    } else {
+      sg = 2 * l > nl;
+      lp = sg ? nl - l : l;
+    }
+  }
+  int tile = lp * ntx + p / kp;
+  if (2 * kx == n1) {                              // the last tile, or beside kx = 0
+    p = 0;
+    tile = lp ? lp * ntx : ntx * nlp;
+    if (lp) sg = 1;
+  }
+  const int i = p % kp, c = i / 4 * 8 + sg * 4 + i % 4;
+  return tile * 2 * zw + c / 8 * 16 + h * 8 + c % 8;
+}
+
 // Words between the planes of a packed spectrum: an odd multiple of 16 (256
 // bytes), so that a z column's values go to all memory channels in turn.  At
 // 64^3 whole rows alone are 32 KB per plane, one channel for a whole column:
@@ -345,7 +378,8 @@ constexpr int y_lanes(int n1, int nl, int ntx) {
 // LDS: exchange buffer E and plane buffer PL (one shared buffer, with more
 // barriers, where both together would exceed LDSCAP: the default leaves room
 // for two workgroups per CU, the stress transform's for four at 64 x 64).
-template <int N1, int N2, int LDSCAP = 80 * 1024, bool FEWREGS = false> struct StepPlane {
+// YINV: the kernel also takes the y lines from layout B to A (line_inv).
+template <int N1, int N2, int LDSCAP = 80 * 1024, bool FEWREGS = false, bool YINV = false> struct StepPlane {
   static constexpr bool ROWS = N2 > 1;
   static constexpr int NL = ROWS ? N2 / 2 : 1;
   using LX = Line<N1>;
@@ -361,7 +395,7 @@ template <int N1, int N2, int LDSCAP = 80 * 1024, bool FEWREGS = false> struct S
   static constexpr int GX = PX < QX ? PX : QX;
   static constexpr int EXW = N1 + N1 / GX + 1;
   static constexpr int EYW = NL | 1;
-  static constexpr int ESIZE = imax(NL * EXW, PY > 1 ? N1 * EYW : 1);
+  static constexpr int ESIZE = imax(NL * EXW, PY > 1 || YINV ? N1 * EYW : 1);
   static constexpr int PLS = N1;                    // row stride in PL
   static constexpr int PSIZE = NL * PLS;
   static constexpr bool ALIAS = (ESIZE + PSIZE + N1 + NL) * 16 > LDSCAP;
@@ -372,9 +406,10 @@ template <int N1, int N2, int LDSCAP = 80 * 1024, bool FEWREGS = false> struct S
   // left (FEWREGS: it has not; a smaller LDSCAP is for launches whose
   // workgroups share a CU, where registers decide how many fit)
   static constexpr bool TWREG =
-      !FEWREGS && LDSCAP >= 80 * 1024 && TwRegs<LX, true>::COUNT <= 12 && TwRegs<LY, false>::COUNT <= 8;
+      !FEWREGS && LDSCAP >= 80 * 1024 && TwRegs<LX, true>::COUNT <= 12 &&
+      (YINV ? !ROWS || TwRegs<LX, true>::COUNT + TwRegs<LY, YINV>::COUNT <= 16 : TwRegs<LY, false>::COUNT <= 8);
   using TwX = std::conditional_t<TWREG, TwRegs<LX, true>, TwTable<LX>>;
-  using TwY = std::conditional_t<TWREG, TwRegs<LY, false>, TwTable<LY>>;
+  using TwY = std::conditional_t<TWREG, TwRegs<LY, YINV>, TwTable<LY>>;
   static constexpr int TWN = TWREG ? 1 : N1 + NL;   // LDS words of the tables
   static_assert(N1 % 2 == 0, "the first grid dimension must be even");
   static_assert(N2 == 1 || N2 % 4 == 0, "the second grid dimension must be 1 or a multiple of 4");
@@ -944,6 +979,204 @@ __global__ void __launch_bounds__(StepZ<N3>::NT) k_step_z(const StepTask* __rest
     }
     a.y *= sg;
     if (act && !(h && sl.o[0] == sl.o[1]) && (MODE != Z_SYM || tz + P * r < np)) st16(arr, ob + P * r * pb, a);
+  }
+}
+
+// ----------------------------------------------------------------------------
+// A whole sweep of a grid with N3 = 1 (1D and 2D cells) in one launch: one
+// workgroup per task keeps the contour field, the factors of the block and the
+// spectra in registers and LDS, and writes each point to the slab.  Nothing
+// passes between workgroups, where the step kernels take four launches per
+// contour step.  Two teams of a plane's threads: in the first convolution team
+// 0 does the full step and team 1 the first half step; in the second, team 1
+// does the other half step, then the Richardson sum, and hands q to team 0.
+// Reciprocal-space factor on packed rows (at StepPlane): with a = C(kx,l), m =
+// C*(-kx,-l), w = exp(-2 pi i l / N2) and s, d the half sum and difference of
+// the factors at ky = l and l + NL, split, product and merge are
+//   C'(kx,l) = (s + d Im w) a + i d Re w m,
+// two real numbers per packed column, held in registers while the block lasts.
+// Bound by the latency of its chain of line transforms (four per step), LDS
+// exchanges and nine barriers (1D: two).  density() + scf_stress() with 100
+// steps, before (four launches per step) and now: 32 points 1260 -> 415 us,
+// 48 x 48 1844 -> 1107 us.
+// ----------------------------------------------------------------------------
+template <int N1, int N2> struct SweepPlane {
+  using SP = StepPlane<N1, N2, 160 * 1024, false, true>;
+  static constexpr int NT = 2 * SP::NT;
+  // both teams' buffers in one workgroup's LDS: edges to 64
+  static constexpr bool OK = NT <= 1024 && !SP::ALIAS && 2 * SP::LDS <= 160 * 1024;
+};
+
+template <int N1, int N2>
+__global__ void __launch_bounds__((SweepPlane<N1, N2>::NT))
+k_sweep_plane(const StepTask* __restrict__ tasks, int last, const double2* __restrict__ tw1g,
+              const double2* __restrict__ twlg, const double2* __restrict__ tw2g) {
+  using SP = typename SweepPlane<N1, N2>::SP;
+  using LX = typename SP::LX;
+  using LY = typename SP::LY;
+  constexpr int QX = SP::QX, QY = SP::QY, PY = SP::PY, UY = SP::UY, PX = SP::PX, UX = SP::UX, NL = SP::NL;
+  constexpr int ZW = StepZ<1>::ZW;
+  __shared__ double2 TWS[SP::TWN];
+  __shared__ double2 EB[2][SP::EBUF];
+  __shared__ double2 PB[2][SP::PBUF];
+  const int team = threadIdx.x / SP::NT, tid = threadIdx.x % SP::NT;
+  double2* const E = EB[team];
+  double2* const PL = PB[team];
+  const StepTask& t = tasks[blockIdx.x];
+  const int jend = t.jend < last + t.jofs ? t.jend : last + t.jofs;   // launches 0 .. last
+  if (t.skip || t.jbeg > jend) return;
+  const typename SP::Roles R(tid);
+  typename SP::Roles R1 = R;         // the second convolution: team 0 only meets the barriers
+  if (team == 0) R1.xact = R1.yact = false;
+  typename SP::Tw tw;
+  tw.load(tw1g, twlg, TWS, R, tid);
+  double2 q[QX], e1[QX], e2[QX];
+#pragma unroll
+  for (int r = 0; r < QX; ++r) q[r] = e1[r] = e2[r] = make_double2(0.0, 0.0);
+  {
+    const int s_in = task_in(t, t.jbeg);
+    const int sl = t.slab ? task_slot(t, s_in) : -1;
+    double* qin = sl >= 0 ? t.slab + (long)sl * t.fm : nullptr;
+    if (R.xact) {
+      if (t.init_one) {
+#pragma unroll
+        for (int r = 0; r < QX; ++r) q[r] = make_double2(1.0, SP::ROWS ? 1.0 : 0.0);
+      } else {
+        SP::get_all(t.start ? t.start : qin, R, q);
+      }
+      if (qin && team == 0 && (t.init_one || t.start)) {
+#pragma unroll
+        for (int r = 0; r < QX; ++r) SP::put(qin, R, r, q[r]);
+      }
+    }
+  }
+  SP::Tw::sync();
+  // factors of the spectrum's points of this thread (2D: y role, layout B over
+  // l; 1D: x role, layout B over kx), of the team's convolution
+  double fa[SP::ROWS ? UY : UX][SP::ROWS ? PY : PX];
+  double fb[SP::ROWS ? UY : 1][SP::ROWS ? PY : 1];
+  const auto conv = [&](double2 (&a)[1][QX], const typename SP::Roles& W) {
+    if constexpr (SP::ROWS) {
+      double2 h[1][UY][PY], c[1][QY];
+      SP::fwd(a, h, E, PL, tw, W);
+      wave_sync();
+      if (W.yact) {
+#pragma unroll
+        for (int u = 0; u < UY; ++u)
+          if (LY::has(W.yt, u)) {
+#pragma unroll
+            for (int k2 = 0; k2 < PY; ++k2) E[W.ey(LY::at(W.yt, u, k2))] = h[0][u][k2];
+          }
+      }
+      __syncthreads();
+      if (W.yact) {
+        const int other = (W.yk ? N1 - W.yk : 0) * SP::EYW;
+#pragma unroll
+        for (int u = 0; u < UY; ++u)
+          if (LY::has(W.yt, u)) {
+#pragma unroll
+            for (int k2 = 0; k2 < PY; ++k2) {
+              const int l = LY::at(W.yt, u, k2);
+              const double2 o = E[other + (l ? NL - l : 0)], v = h[0][u][k2];
+              h[0][u][k2] = make_double2(mad(fa[u][k2], v.x, fb[u][k2] * o.y),
+                                         mad(fa[u][k2], v.y, fb[u][k2] * o.x));
+            }
+          }
+      }
+      __syncthreads();
+      line_inv<LY, +1, 1>(h, c, E, [&](int, int i) { return W.ey(i); }, W.yt, tw.y, W.yact);
+      if (W.yact) {
+#pragma unroll
+        for (int r = 0; r < QY; ++r) PL[(W.yt + PY * r) * SP::PLS + W.yk] = c[0][r];
+      }
+      __syncthreads();
+      SP::inv_x(a, E, PL, tw, W);
+    } else {
+      double2 b[1][UX][PX];
+      const auto ex = [&](int, int i) { return W.ex(i); };
+      line_fwd<LX, -1, 1>(a, b, E, ex, W.xt, tw.x, W.xact);
+#pragma unroll
+      for (int u = 0; u < UX; ++u)
+        if (W.xact && LX::has(W.xt, u)) {
+#pragma unroll
+          for (int k2 = 0; k2 < PX; ++k2) b[0][u][k2] = cscale(b[0][u][k2], fa[u][k2]);
+        }
+      line_inv<LX, +1, 1>(b, a, E, ex, W.xt, tw.x, W.xact);
+    }
+  };
+  const double i3 = 1.0 / 3.0;
+  double2* const X = PB[0] + R.xl * SP::PLS + R.xt;   // q1, then q: a thread's own words of its row
+  int block = -1;
+  for (int j = t.jbeg; j < jend; ++j) {
+    const int b = task_block(t, j);
+    const int so = t.slab ? task_slot(t, task_out(t, j)) : -1;
+    if (b != block) {
+      block = b;
+      const double* kf = team ? task_k2(t, b) : task_k1(t, b);
+      if (R.xact) {
+        SP::get_all(task_e1(t, b), R, e1);
+        SP::get_all(task_e2(t, b), R, e2);
+      }
+      if constexpr (SP::ROWS) {
+        if (R.yact) {
+#pragma unroll
+          for (int u = 0; u < UY; ++u)
+            if (LY::has(R.yt, u)) {
+#pragma unroll
+              for (int k2 = 0; k2 < PY; ++k2) {
+                const int l = LY::at(R.yt, u, k2);
+                const double f0 = kf[z_factor_at(R.yk, l, 0, N1, NL, ZW)];
+                const double f1 = kf[z_factor_at(R.yk, l, 1, N1, NL, ZW)];
+                const double2 w = tw2g[l];
+                fa[u][k2] = 2.0 * mad(f0 - f1, w.y, f0 + f1);    // k_step_z's factor 4
+                fb[u][k2] = 2.0 * (f0 - f1) * w.x;
+              }
+            }
+        }
+      } else if (R.xact) {
+#pragma unroll
+        for (int u = 0; u < UX; ++u)
+          if (LX::has(R.xt, u)) {
+#pragma unroll
+            for (int k2 = 0; k2 < PX; ++k2)
+              fa[u][k2] = kf[z_factor_at(LX::at(R.xt, u, k2), 0, 0, N1, 1, ZW)];
+          }
+      }
+    }
+    double2 a[1][QX];
+#pragma unroll
+    for (int r = 0; r < QX; ++r) {
+      const double2 f = team ? e2[r] : e1[r];
+      a[0][r] = make_double2(f.x * q[r].x, f.y * q[r].y);
+    }
+    conv(a, R);
+#pragma unroll
+    for (int r = 0; r < QX; ++r) a[0][r] = make_double2(e1[r].x * a[0][r].x, e1[r].y * a[0][r].y);
+    if (team == 0 && R.xact) {
+#pragma unroll
+      for (int r = 0; r < QX; ++r) X[PX * r] = a[0][r];
+    }
+    if constexpr (!SP::ROWS) __syncthreads();
+    conv(a, R1);
+    if (R1.xact) {
+#pragma unroll
+      for (int r = 0; r < QX; ++r) {
+        const double2 q1 = X[PX * r];
+        const double2 q2 = make_double2(e2[r].x * a[0][r].x, e2[r].y * a[0][r].y);
+        q[r] = make_double2(div_by(4.0 * q2.x - q1.x, 3.0, i3), div_by(4.0 * q2.y - q1.y, 3.0, i3));
+        X[PX * r] = q[r];
+      }
+      if (so >= 0) {
+        double* qo = t.slab + (long)so * t.fm;
+#pragma unroll
+        for (int r = 0; r < QX; ++r) SP::put(qo, R, r, q[r]);
+      }
+    }
+    __syncthreads();
+    if (team == 0 && R.xact) {
+#pragma unroll
+      for (int r = 0; r < QX; ++r) q[r] = X[PX * r];
+    }
   }
 }
 

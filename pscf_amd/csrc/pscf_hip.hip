@@ -139,6 +139,7 @@ const double2* twiddles(int n) {
 // ------------------------------------------------------- kernel dispatch
 using StepPlaneFn = void (*)(const StepTask*, int, const double2*, const double2*);
 using StepZFn = void (*)(const StepTask*, int, int, int, const double2*, const double2*);
+using SweepFn = void (*)(const StepTask*, int, const double2*, const double2*, const double2*);
 using R2CFn = void (*)(const double*, long, double2*, long, const double2*, const double2*,
                        const int*, int);
 using C2RFn = void (*)(const double2*, long, double*, long, double, const double2*, const double2*);
@@ -157,6 +158,8 @@ struct PlaneSet {
   // [adjoint sweeps]: k_step_a with one and two workgroups per plane, k_step_c,
   // and k_step_c with shared exchange/plane LDS (wide launches)
   StepPlaneFn a1[2] = {}, a[2] = {}, c[2] = {}, c_wide[2] = {};
+  SweepFn sweep = nullptr;    // whole sweeps of grids with N3 = 1, where compiled
+  int nt_sweep = 0;
   R2CFn r2c = nullptr;
   R2CColsFn r2c_cols = nullptr;   // register-line XY pass of scf_stress's transforms
   C2RFn c2r = nullptr;
@@ -194,6 +197,10 @@ PlaneSet make_plane() {
   constexpr int wpe = A >= 48 && A <= 64 && B >= 48 && B <= 64 ? 4 : 1;
   s.c_wide[0] = k_step_c<A, B, false, 40 * 1024, wpe>;
   s.c_wide[1] = k_step_c<A, B, true, 40 * 1024, wpe>;
+  if constexpr (SweepPlane<A, B>::OK) {
+    s.sweep = k_sweep_plane<A, B>;
+    s.nt_sweep = SweepPlane<A, B>::NT;
+  }
   s.r2c = k_plane_r2c<A, B>;
   s.r2c_cols = k_plane_r2c_cols<A, B>;
   s.c2r = k_plane_c2r<A, B>;
@@ -722,11 +729,18 @@ void launch_step_a(const Grid& g, const StepTask* tasks, int ntask, int j, bool 
 }
 
 // --------------------------------------------------- contour sweeps
-// Advance the given sweep tasks through all their steps (4 launches per step).
+// Advance the given sweep tasks through all their steps: one launch where the
+// grid is one plane (k_sweep_plane), else 4 launches per step.
 // With `ev` (2 (4 max_ns + 1) events) every launch records a pair of events at
 // its kernel's start and end, for per-kernel timing.
 void run_sweeps(const Grid& g, const StepTask* d_tasks, int ntask, int max_ns, hipStream_t s,
                 hipEvent_t* ev = nullptr) {
+  if (g.n3 == 1 && g.pl->sweep && !ev) {
+    hipLaunchKernelGGL(g.pl->sweep, dim3(ntask), dim3(g.pl->nt_sweep), 0, s, d_tasks, max_ns, g.tw1, g.twl,
+                       g.tw2);
+    HIPCHK(hipGetLastError());
+    return;
+  }
   int e = 0;
   auto t0 = [&] { return ev ? ev[e] : nullptr; };
   auto t1 = [&] { return ev ? ev[e + 1] : nullptr; };
