@@ -208,17 +208,32 @@ __host__ __device__ __forceinline__ int sym_weight(int sym, int n3, int u) {
   const int np = sym_planes(sym, n3);
   return ((sym & SYM_T) ? 2 : 1) * ((sym & SYM_R) && u != 0 && u != np - 1 ? 2 : 1);
 }
-// grid index of the stored point with the value of grid point g (planes n1 x n2)
-__host__ __device__ __forceinline__ long sym_point(int sym, int n1, int n2, int n3, long g) {
-  int x = (int)(g % n1), y = (int)(g / n1 % n2), u;
-  const int op = sym_source(sym, n3, (int)(g / ((long)n1 * n2)), u);
+// the point of a plane that operation `op` takes to (x, y)
+__host__ __device__ __forceinline__ int sym_in_plane(int op, int n1, int n2, int x, int y) {
   if (op & 2) x = x >= n1 / 2 ? x - n1 / 2 : x + n1 / 2;
   if (op & 4) y = y >= n2 / 2 ? y - n2 / 2 : y + n2 / 2;
   if (op & 1) {
     x = x ? n1 - x : 0;
     y = y ? n2 - y : 0;
   }
-  return x + n1 * (y + (long)n2 * u);
+  return x + n1 * y;
+}
+// grid index of the stored point with the value of grid point g (planes n1 x n2)
+__host__ __device__ __forceinline__ long sym_point(int sym, int n1, int n2, int n3, long g) {
+  int u;
+  const int op = sym_source(sym, n3, (int)(g / ((long)n1 * n2)), u);
+  return sym_in_plane(op, n1, n2, (int)(g % n1), (int)(g / n1 % n2)) + (long)n1 * n2 * u;
+}
+// a point that the symmetry gives the value of grid point g, so that a field
+// is symmetric if all these pairs are equal: the stored point, or on the first
+// and last stored plane, which z -> -z maps onto themselves, the image there;
+// g itself on the others
+__host__ __device__ __forceinline__ long sym_partner(int sym, int n1, int n2, int n3, long g) {
+  const int z = (int)(g / ((long)n1 * n2)), np = sym_planes(sym, n3);
+  if (z >= np) return sym_point(sym, n1, n2, n3, g);
+  if (!(sym & SYM_R) || (z != 0 && z != np - 1)) return g;
+  const int op = sym >> (z != 0 && (sym & SYM_T) ? 8 : 5) & 7;
+  return sym_in_plane(op, n1, n2, (int)(g % n1), (int)(g / n1 % n2)) + (long)n1 * n2 * z;
 }
 // flip the sign of v where bit 31 of m is set
 __device__ __forceinline__ double sign_flip(double v, int m) {
@@ -862,13 +877,13 @@ template <int N3> struct StepZ {
   }
 };
 
-enum { Z_PLAIN = 0, Z_ADJ = 1, Z_SYM = 2 };
+enum { Z_PLAIN = 0, Z_ADJ = 1, Z_SYM = 2 };    // flags
 template <int N1, int N3, int MODE>
 __global__ void __launch_bounds__(StepZ<N3>::NT) k_step_z(const StepTask* __restrict__ tasks, int jl, int N2,
                                                        int kind, const double2* __restrict__ tw2g,
                                                        const double2* __restrict__ tw3g) {
   using SZ = StepZ<N3>;
-  constexpr bool ADJ = MODE == Z_ADJ;
+  constexpr bool ADJ = (MODE & Z_ADJ) != 0, SYM = (MODE & Z_SYM) != 0;
   using L = typename SZ::L;
   constexpr int P = SZ::P, Q = SZ::Q, U = SZ::U, ZW = SZ::ZW;
   constexpr int N1H = N1 / 2 + 1;
@@ -887,22 +902,22 @@ __global__ void __launch_bounds__(StepZ<N3>::NT) k_step_z(const StepTask* __rest
   const int io = h ? sl.o[1] : sl.o[0];            // this lane's packed column
   const unsigned pb = 16 * plane_words(N1, nl);    // bytes per plane
   const unsigned ob = 16 * io + tz * pb;
-  const int np = MODE == Z_SYM ? sym_planes(t.sym, N3) : N3;
+  const int np = SYM ? sym_planes(t.sym, N3) : N3;
   const int b = task_block(t, j);
   double2* arr = kind == 0 ? (job == 0 ? t.A : t.B) : t.C;
   const double* kf = kind == 0 && job == 0 ? task_k1(t, b) : task_k2(t, b);
   double2 v[1][Q], wl = make_double2(1.0, 0.0);
   double f[U][P];
-  int op[MODE == Z_SYM ? Q : 1];
+  int op[SYM ? Q : 1];
 #pragma unroll
   for (int r = 0; r < Q; ++r) {
     v[0][r] = make_double2(0.0, 0.0);
-    if constexpr (MODE == Z_SYM) op[r] = 0;
+    if constexpr (SYM) op[r] = 0;
   }
   if (act) {
 #pragma unroll
     for (int r = 0; r < Q; ++r) {
-      if constexpr (MODE == Z_SYM) {
+      if constexpr (SYM) {
         int u;
         op[r] = sym_source(t.sym, N3, tz + P * r, u);
         v[0][r] = ld16(arr, 16 * io + u * pb);
@@ -941,7 +956,7 @@ __global__ void __launch_bounds__(StepZ<N3>::NT) k_step_z(const StepTask* __rest
       if (h) v[0][r] = oth;
     }
   }
-  if constexpr (MODE == Z_SYM) {
+  if constexpr (SYM) {
     // the operation from the stored plane, at this lane's column (kx, ky)
     const int sx = sl.kx << 31, sy = (sl.l + h * nl) << 31;
 #pragma unroll
@@ -978,7 +993,7 @@ __global__ void __launch_bounds__(StepZ<N3>::NT) k_step_z(const StepTask* __rest
       a = cfma(iw, csub(a, oth), cadd(a, oth));
     }
     a.y *= sg;
-    if (act && !(h && sl.o[0] == sl.o[1]) && (MODE != Z_SYM || tz + P * r < np)) st16(arr, ob + P * r * pb, a);
+    if (act && !(h && sl.o[0] == sl.o[1]) && (!SYM || tz + P * r < np)) st16(arr, ob + P * r * pb, a);
   }
 }
 

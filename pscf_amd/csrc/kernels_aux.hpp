@@ -142,16 +142,17 @@ __global__ void __launch_bounds__(NTA) k_make_propg(double ds, double b, const d
   }
 }
 
-// nf fields (stride m each) between the grid order and the sweeps' packed order
+// nf fields between the grid order (mg points each) and the sweeps' packed order
+// (m each)
 __global__ void __launch_bounds__(NTA) k_unpack(const double* __restrict__ packed, long m, int nf, int n1,
                                                 int n2, double* __restrict__ grid) {
   for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < m * nf; i += (long)gridDim.x * NTA)
     grid[i / m * m + unpack_index(i % m, n1, n2)] = packed[i];
 }
-__global__ void __launch_bounds__(NTA) k_pack(const double* __restrict__ grid, long m, int nf, int n1, int n2,
-                                              double* __restrict__ packed) {
+__global__ void __launch_bounds__(NTA) k_pack(const double* __restrict__ grid, long mg, long m, int nf, int n1,
+                                              int n2, double* __restrict__ packed) {
   for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < m * nf; i += (long)gridDim.x * NTA)
-    packed[i] = grid[i / m * m + unpack_index(i % m, n1, n2)];
+    packed[i] = grid[i / m * mg + unpack_index(i % m, n1, n2)];
 }
 
 // ----------------------------------------------------------------------------
@@ -312,12 +313,13 @@ __global__ void __launch_bounds__(NTA) k_partial_qlogq(const double* __restrict_
 // Adjoint support.
 // k_simpson_lam: per block b of a chain (blockIdx.y), workgroup partials of
 //   T_b = ds_b/3 sum_r lam_mon(b)(r) [qf qr(ibgn) + qf qr(iend) + 4 sum_odd + 2 sum_even]
-// i.e. the block's Simpson density weighted by lam (part[b*gridDim.x + x]).
+// i.e. the block's Simpson density weighted by lam (part[b*gridDim.x + x]);
+// sym, n3, plane: as k_partial_sum.
 // ----------------------------------------------------------------------------
 __global__ void __launch_bounds__(NTA) k_simpson_lam(const double* __restrict__ qf,
                                                      const double* __restrict__ qr, long m,
-                                                     SimpsonArgs a, const double* __restrict__ lam,
-                                                     double* __restrict__ part) {
+                                                     SimpsonArgs a, const double* __restrict__ lam, int sym,
+                                                     int n3, long plane, double* __restrict__ part) {
   __shared__ double red[NTA];
   const int b = blockIdx.y;
   const int ibgn = a.bnd[b], iend = a.bnd[b + 1];
@@ -328,7 +330,7 @@ __global__ void __launch_bounds__(NTA) k_simpson_lam(const double* __restrict__ 
     acc += qf[(long)iend * m + r] * qr[(long)iend * m + r];
     for (int jj = ibgn + 1; jj <= iend - 1; jj += 2) acc += 4.0 * qf[(long)jj * m + r] * qr[(long)jj * m + r];
     for (int jj = ibgn + 2; jj <= iend - 2; jj += 2) acc += 2.0 * qf[(long)jj * m + r] * qr[(long)jj * m + r];
-    tot += lm[r] * acc;
+    tot += sym ? lm[r] * acc * sym_weight(sym, n3, (int)(r / plane)) : lm[r] * acc;
   }
   const double s = block_sum(tot * a.ds[b] / 3.0, red);
   if (threadIdx.x == 0) part[(long)b * gridDim.x + blockIdx.x] = s;
@@ -373,13 +375,14 @@ __global__ void __launch_bounds__(NTA) k_block_rho(const double* __restrict__ bl
   }
 }
 
-// workgroup partials of sum x*y
+// workgroup partials of sum x*y (sym, n3, plane: as k_partial_sum)
 __global__ void __launch_bounds__(NTA) k_partial_dot(const double* __restrict__ x,
-                                                     const double* __restrict__ y, long n,
-                                                     double* __restrict__ part) {
+                                                     const double* __restrict__ y, long n, int sym, int n3,
+                                                     long plane, double* __restrict__ part) {
   __shared__ double red[NTA];
   double acc = 0.0;
-  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < n; i += (long)gridDim.x * NTA) acc += x[i] * y[i];
+  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < n; i += (long)gridDim.x * NTA)
+    acc += sym ? x[i] * y[i] * sym_weight(sym, n3, (int)(i / plane)) : x[i] * y[i];
   const double s = block_sum(acc, red);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
@@ -448,6 +451,34 @@ __global__ void __launch_bounds__(NTA) k_sym_check(const double* __restrict__ f,
     const double* g = f + i / (m - m0) * m;
     const long p = m0 + i % (m - m0);
     bad = bad || !(fabs(g[p] - g[sym_point(sym, n1, n2, n3, p)]) <= tol);
+  }
+  if (bad) flag[0] = epoch;
+}
+
+// The check for fields given on the grid, which need not have the symmetry
+// anywhere: every pair of sym_partner, against tol times the fields' largest
+// modulus.  Workgroup maxima of |x|, then the check (part: np maxima).
+__global__ void __launch_bounds__(NTA) k_partial_absmax(const double* __restrict__ x, long n,
+                                                        double* __restrict__ part) {
+  __shared__ double red[NTA];
+  double v = 0.0;
+  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < n; i += (long)gridDim.x * NTA) v = fmax(v, fabs(x[i]));
+  red[threadIdx.x] = v;
+  __syncthreads();
+  if (threadIdx.x) return;
+  for (int i = 1; i < NTA; ++i) v = fmax(v, red[i]);
+  part[blockIdx.x] = v;
+}
+__global__ void __launch_bounds__(NTA) k_sym_check_grid(const double* __restrict__ f, int nf, int sym, int n1,
+                                                        int n2, int n3, const double* __restrict__ part, int np,
+                                                        double tol, double epoch, double* __restrict__ flag) {
+  const long m = (long)n1 * n2 * n3;
+  double big = 0.0;
+  for (int i = 0; i < np; ++i) big = fmax(big, part[i]);
+  bool bad = false;
+  for (long i = blockIdx.x * (long)NTA + threadIdx.x; i < m * nf; i += (long)gridDim.x * NTA) {
+    const double* g = f + i / m * m;
+    bad = bad || !(fabs(g[i % m] - g[sym_partner(sym, n1, n2, n3, i % m)]) <= tol * big);
   }
   if (bad) flag[0] = epoch;
 }
