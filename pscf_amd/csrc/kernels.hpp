@@ -856,38 +856,53 @@ __global__ void __launch_bounds__((StepPlane<N1, N2>::NT)) k_plane_r2c_cols(
 // planes; loads a column from its stored planes (each up to four times, from
 // the cache) and stores those.
 // ----------------------------------------------------------------------------
-template <int N3> struct StepZ {
-  using L = Line<N3>;
+// LEN: points of the lines, N3 or (Z_HALF) N3/2.
+template <int N3, int LEN = N3> struct StepZ {
+  using L = Line<LEN>;
   static constexpr int P = L::P, Q = L::Q, U = L::U;
-  static constexpr int ZW = imax(1, plan_zl(N3) / P / 8) * 8;   // slots per workgroup
+  static constexpr int ZW = imax(1, plan_zl(N3) / Line<N3>::P / 8) * 8;   // slots per workgroup
   static constexpr int NT = clampnt(round64(2 * ZW * P));
   static constexpr int NTC = clampnt(round64(ZW * P));  // of k_zfwd_cols
   // twiddles in registers where they are few, else a table in LDS
   static constexpr bool TWREG = TwRegs<L, true>::COUNT <= 12;
   using Tw = std::conditional_t<TWREG, TwRegs<L, true>, TwTable<L>>;
-  static constexpr int TWN = TWREG ? 1 : N3;
+  static constexpr int TWN = TWREG ? 1 : LEN;
   template <int T> static __device__ __forceinline__ void load_tw(Tw& tw, const double2* __restrict__ g,
                                                                   double2* lds, int tz, int tid) {
     if constexpr (TWREG) {
       tw.load(g, tz);
     } else {
-      stage_tw<N3, T>(lds, g, tid);
+      stage_tw<LEN, T>(lds, g, tid);
       tw.tw = lds;
     }
   }
 };
 
-enum { Z_PLAIN = 0, Z_ADJ = 1, Z_SYM = 2 };    // flags
+enum { Z_PLAIN = 0, Z_ADJ = 1, Z_SYM = 2, Z_HALF = 4 };    // flags
+// Z_HALF (with Z_SYM): the translation z -> z + N3/2 without a rotation in the
+// plane (body, face and base centring).  A column is then periodic or
+// antiperiodic over half the edge, and only its even or its odd kz are not
+// zero: lines of N3/2 points, twiddled by w_N3^z where antiperiodic.
+// Half the points, LDS words and butterflies of the whole lines; density() +
+// scf_stress() before and now: gyroid 64^3 6125 -> 5649 us, 96^3 13640 ->
+// 12250 us, 32 body-centred 32^3 fields 7293 -> 6652 us.  Reverse-mode sweeps
+// keep whole lines: their kept spectra need the zeros too.
+constexpr bool sym_half(int sym) { return (sym & SYM_T) != 0 && !(sym >> 2 & 1); }
+constexpr bool z_half_ok(int n3) { return n3 % 2 == 0 && line_plan(n3 / 2).p > 0; }
+// twiddle tables of length n, then n/2 (Z_HALF's lines)
+constexpr int z_tables(int n3) { return n3 + n3 / 2; }
 template <int N1, int N3, int MODE>
-__global__ void __launch_bounds__(StepZ<N3>::NT) k_step_z(const StepTask* __restrict__ tasks, int jl, int N2,
+__global__ void __launch_bounds__((StepZ<N3, (MODE & Z_HALF) ? N3 / 2 : N3>::NT)) k_step_z(const StepTask* __restrict__ tasks, int jl, int N2,
                                                        int kind, const double2* __restrict__ tw2g,
                                                        const double2* __restrict__ tw3g) {
-  using SZ = StepZ<N3>;
+  constexpr bool HALF = (MODE & Z_HALF) != 0;
+  constexpr int NZ = HALF ? N3 / 2 : N3;
+  using SZ = StepZ<N3, NZ>;
   constexpr bool ADJ = (MODE & Z_ADJ) != 0, SYM = (MODE & Z_SYM) != 0;
   using L = typename SZ::L;
   constexpr int P = SZ::P, Q = SZ::Q, U = SZ::U, ZW = SZ::ZW;
   constexpr int N1H = N1 / 2 + 1;
-  __shared__ double2 E[N3 > 1 ? 2 * N3 * ZW : 1];
+  __shared__ double2 E[NZ > 1 ? 2 * NZ * ZW : 1];
   __shared__ double2 TWS[SZ::TWN];
   const int tid = threadIdx.x, hc = tid % (2 * ZW), tz = tid / (2 * ZW);
   const int h = z_lane_h(hc), c = z_lane_slot(hc);
@@ -906,6 +921,8 @@ __global__ void __launch_bounds__(StepZ<N3>::NT) k_step_z(const StepTask* __rest
   const int b = task_block(t, j);
   double2* arr = kind == 0 ? (job == 0 ? t.A : t.B) : t.C;
   const double* kf = kind == 0 && job == 0 ? task_k1(t, b) : task_k2(t, b);
+  // antiperiodic columns (HALF): odd kz
+  const int odd = HALF ? ((t.sym & 8 ? sl.kx : 0) ^ (t.sym & 16 ? sl.l + h * nl : 0)) & 1 : 0;
   double2 v[1][Q], wl = make_double2(1.0, 0.0);
   double f[U][P];
   int op[SYM ? Q : 1];
@@ -931,11 +948,19 @@ __global__ void __launch_bounds__(StepZ<N3>::NT) k_step_z(const StepTask* __rest
     for (int u = 0; u < U; ++u)
       if (L::has(tz, u)) {
 #pragma unroll
-        for (int k2 = 0; k2 < P; ++k2) f[u][k2] = kf[k0 + (P * u + Q * k2) * kz];
+        for (int k2 = 0; k2 < P; ++k2) {
+          if constexpr (HALF) f[u][k2] = 2.0 * kf[k0 - tz * kz + (2 * (tz + P * u + Q * k2) + odd) * kz];
+          else f[u][k2] = kf[k0 + (P * u + Q * k2) * kz];
+        }
       }
   }
+  double2 wz[HALF ? Q : 1];
+  if constexpr (HALF) {
+#pragma unroll
+    for (int r = 0; r < Q; ++r) wz[r] = odd && act ? tw3g[tz + P * r] : make_double2(1.0, 0.0);
+  }
   typename SZ::Tw tw;
-  SZ::template load_tw<SZ::NT>(tw, tw3g, TWS, tz, tid);
+  SZ::template load_tw<SZ::NT>(tw, HALF ? tw3g + N3 : tw3g, TWS, tz, tid);
   if constexpr (!SZ::TWREG) __syncthreads();
   // split: v = 2 F(ky = l + h NL) = a + m + (-1)^h w^l (a - m)/i with a =
   // C(kx,l), m = C*(-kx,-l), written in the sums and differences of this
@@ -964,6 +989,7 @@ __global__ void __launch_bounds__(StepZ<N3>::NT) k_step_z(const StepTask* __rest
       const int m = ((op[r] & 2) ? sx : 0) ^ ((op[r] & 4) ? sy : 0);
       v[0][r].x = sign_flip(v[0][r].x, m);
       v[0][r].y = sign_flip(v[0][r].y, m ^ (op[r] << 31));
+      if constexpr (HALF) v[0][r] = cmul(v[0][r], wz[r]);
     }
   }
   double2 w[1][U][P];
@@ -988,6 +1014,7 @@ __global__ void __launch_bounds__(StepZ<N3>::NT) k_step_z(const StepTask* __rest
 #pragma unroll
   for (int r = 0; r < Q; ++r) {
     double2 a = v[0][r];
+    if constexpr (HALF) a = cmul(a, cconj(wz[r]));
     if (rows) {
       const double2 oth = lane_swap(a);
       a = cfma(iw, csub(a, oth), cadd(a, oth));

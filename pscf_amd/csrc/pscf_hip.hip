@@ -127,11 +127,12 @@ const double2* twiddles(int n) {
   std::lock_guard<std::mutex> lk(g_tw_mutex);
   auto it = g_tw.find(n);
   if (it != g_tw.end()) return it->second;
-  std::vector<double2> h(n);
+  std::vector<double2> h(z_tables(n));      // of length n, then n/2
   host_twiddles(n, h.data());
+  if (n > 1) host_twiddles(n / 2, h.data() + n);
   double2* d = nullptr;
-  HIPCHK(hipMalloc((void**)&d, sizeof(double2) * n));
-  HIPCHK(hipMemcpy(d, h.data(), sizeof(double2) * n, hipMemcpyHostToDevice));
+  HIPCHK(hipMalloc((void**)&d, sizeof(double2) * h.size()));
+  HIPCHK(hipMemcpy(d, h.data(), sizeof(double2) * h.size(), hipMemcpyHostToDevice));
   g_tw[n] = d;
   return d;
 }
@@ -171,6 +172,8 @@ struct ZSet {
   int nt_cols = 0;                // of the stress transform's z kernel
   int zw = 1;                     // their column slots and columns per workgroup
   StepZFn z[4] = {};              // by the flags Z_ADJ, Z_SYM
+  StepZFn z_half = nullptr;       // Z_HALF, where N3/2 has a line plan
+  int nt_half_step = 0;
   ZfftFn half_f = nullptr, half_i = nullptr, full_f = nullptr, full_i = nullptr;
   ZColsFn cols_f = nullptr;       // register-line forward z pass of scf_stress's spectra
 };
@@ -223,6 +226,10 @@ ZSet make_z() {
   if constexpr (C > 1) {
     s.z[Z_SYM] = k_step_z<A, C, Z_SYM>;
     s.z[Z_ADJ | Z_SYM] = k_step_z<A, C, (Z_ADJ | Z_SYM)>;
+    if constexpr (z_half_ok(C)) {
+      s.z_half = k_step_z<A, C, (Z_SYM | Z_HALF)>;
+      s.nt_half_step = StepZ<C, C / 2>::NT;
+    }
   }
   s.half_f = k_zfft<A / 2 + 1, C, -1>;
   s.cols_f = k_zfwd_cols<C>;
@@ -357,14 +364,17 @@ struct Grid {
   // With events (t0, t1), the launch records them at the start and the end of
   // the kernel's execution (hipExtLaunchKernelGGL: no launch gaps included).
   // adj: the tasks are adjoint or recomputed sweeps
-  void step_z(const StepTask* tasks, int ntask, int j, int kind, int jobs, bool adj, hipStream_t s,
+  // half_z: every task's planes allow the half-length z lines (sym_half)
+  void step_z(const StepTask* tasks, int ntask, int j, int kind, int jobs, bool adj, bool half_z, hipStream_t s,
               hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr) const {
     const dim3 grid(z_tiles(n1, nl, zs->zw), ntask, jobs);
-    const StepZFn k = zs->z[(adj ? Z_ADJ : 0) | (sym ? Z_SYM : 0)];
+    const bool half = !adj && half_z && zs->z_half;
+    const StepZFn k = half ? zs->z_half : zs->z[(adj ? Z_ADJ : 0) | (sym ? Z_SYM : 0)];
+    const dim3 nt(half ? zs->nt_half_step : zs->nt_step);
     if (t0)
-      hipExtLaunchKernelGGL(k, grid, dim3(zs->nt_step), 0, s, t0, t1, 0, tasks, j, n2, kind, tw2, tw3);
+      hipExtLaunchKernelGGL(k, grid, nt, 0, s, t0, t1, 0, tasks, j, n2, kind, tw2, tw3);
     else
-      hipLaunchKernelGGL(k, grid, dim3(zs->nt_step), 0, s, tasks, j, n2, kind, tw2, tw3);
+      hipLaunchKernelGGL(k, grid, nt, 0, s, tasks, j, n2, kind, tw2, tw3);
   }
   // launches that need more than two rounds of resident workgroups take the
   // form whose smaller LDS footprint lets more of them reside on a CU at once
@@ -736,7 +746,8 @@ void launch_step_a(const Grid& g, const StepTask* tasks, int ntask, int j, bool 
 // grid is one plane (k_sweep_plane), else 4 launches per step.
 // With `ev` (2 (4 max_ns + 1) events) every launch records a pair of events at
 // its kernel's start and end, for per-kernel timing.
-void run_sweeps(const Grid& g, const StepTask* d_tasks, int ntask, int max_ns, hipStream_t s,
+// half_z: see step_z (the tasks of one launch may be of several systems)
+void run_sweeps(const Grid& g, const StepTask* d_tasks, int ntask, int max_ns, bool half_z, hipStream_t s,
                 hipEvent_t* ev = nullptr) {
   if (g.n3 == 1 && g.pl->sweep && !ev) {
     hipLaunchKernelGGL(g.pl->sweep, dim3(ntask), dim3(g.pl->nt_sweep), 0, s, d_tasks, max_ns, g.tw1, g.twl,
@@ -752,11 +763,11 @@ void run_sweeps(const Grid& g, const StepTask* d_tasks, int ntask, int max_ns, h
     launch_step_a(g, d_tasks, ntask, j, false, s, t0(), t1());
     next();
     if (j == max_ns) break;
-    g.step_z(d_tasks, ntask, j, 0, 2, false, s, t0(), t1());
+    g.step_z(d_tasks, ntask, j, 0, 2, false, half_z, s, t0(), t1());
     next();
     g.step_c(d_tasks, ntask, j, false, s, t0(), t1());
     next();
-    g.step_z(d_tasks, ntask, j, 1, 1, false, s, t0(), t1());
+    g.step_z(d_tasks, ntask, j, 1, 1, false, half_z, s, t0(), t1());
     next();
   }
   HIPCHK(hipGetLastError());
@@ -1140,7 +1151,7 @@ void ck_simpson_rounds(System& S, hipStream_t s) {
   }
   for (int r = 0; r < P.nround; ++r) {
     const StepTask* tk = S.ck_tasks.p + (size_t)r * 2 * nc;
-    run_sweeps(g, tk, 2 * nc, P.len[r], s);
+    run_sweeps(g, tk, 2 * nc, P.len[r], sym_half(g.sym), s);
     for (int c = 0; c < nc; ++c) {
       ChainDev& ch = *S.chains[c];
       const int lo = r * K, hi = std::min((r + 1) * K, ch.ns);
@@ -1367,7 +1378,7 @@ void density_sweeps(System& S, hipStream_t s) {
   ++S.density_gen;
   if (S.profile == 2) {
     ensure_events(S, (size_t)2 * (4 * max_ns + 1));
-    run_sweeps(g, S.tasks.p, S.ntask, max_ns, s, S.ev.data());
+    run_sweeps(g, S.tasks.p, S.ntask, max_ns, sym_half(g.sym), s, S.ev.data());
     return;
   }
   if (S.profile == 1) {
@@ -1377,13 +1388,13 @@ void density_sweeps(System& S, hipStream_t s) {
   if (S.use_graph) {
     if (!S.graph_exec) {
       HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-      run_sweeps(g, S.tasks.p, S.ntask, max_ns, s);
+      run_sweeps(g, S.tasks.p, S.ntask, max_ns, sym_half(g.sym), s);
       HIPCHK(hipStreamEndCapture(s, &S.graph));
       HIPCHK(hipGraphInstantiate(&S.graph_exec, S.graph, nullptr, nullptr, 0));
     }
     HIPCHK(hipGraphLaunch(S.graph_exec, s));
   } else {
-    run_sweeps(g, S.tasks.p, S.ntask, max_ns, s);
+    run_sweeps(g, S.tasks.p, S.ntask, max_ns, sym_half(g.sym), s);
   }
   if (S.profile == 1) HIPCHK(hipEventRecord(S.ev[1], s));
 }
@@ -1750,13 +1761,13 @@ void density_many(System& S, int n, const double* omega, double* rho, double* qo
       if (S.use_graph) {
         if (!Mu.exec) {
           HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-          run_sweeps(g, Mu.tasks.p, nt, Mu.max_ns, s);
+          run_sweeps(g, Mu.tasks.p, nt, Mu.max_ns, sym_half(g.sym), s);
           HIPCHK(hipStreamEndCapture(s, &Mu.graph));
           HIPCHK(hipGraphInstantiate(&Mu.exec, Mu.graph, nullptr, nullptr, 0));
         }
         HIPCHK(hipGraphLaunch(Mu.exec, s));
       } else {
-        run_sweeps(g, Mu.tasks.p, nt, Mu.max_ns, s);
+        run_sweeps(g, Mu.tasks.p, nt, Mu.max_ns, sym_half(g.sym), s);
       }
     }
     for (int i = 0; i < cnt; ++i) density_post(*Mu.cl[i], rho + (size_t)(k0 + i) * nst, s);
@@ -1966,6 +1977,7 @@ struct AdjSweeps {
   int npair = 0;
   int max_ns = 0;
   bool with_k = false;
+  bool half_z = false;                   // every system's planes allow it (step_z)
   int K = 0, nround = 0;
   const int* len = nullptr;              // per round: longest segment
   const StepTask* ck_rec = nullptr;      // per round: ntask recomputation tasks
@@ -1981,16 +1993,16 @@ void run_adj_sweeps(const Grid& g, const AdjSweeps& W, hipStream_t s) {
     if (K > 0) {
       const int r = std::min(j / K, W.nround - 1);
       if (j % K == 0 && j / K < W.nround)
-        run_sweeps(g, W.ck_rec + (size_t)r * nt, nt, W.len[r], s);
+        run_sweeps(g, W.ck_rec + (size_t)r * nt, nt, W.len[r], W.half_z, s);
       tasks = W.ck_adj + (size_t)r * nt;
     }
     launch_step_a(g, tasks, nt, j, true, s);
     if (j >= 1)
       hipLaunchKernelGGL(k_adj_grad, dim3(gb), dim3(256), 0, s, tasks, W.pairs, W.npair, j - 1, g.ms);
     if (j == max_ns) break;
-    g.step_z(tasks, nt, j, 0, 2, true, s);
+    g.step_z(tasks, nt, j, 0, 2, true, false, s);
     g.step_c(tasks, nt, j, true, s);
-    g.step_z(tasks, nt, j, 1, 1, true, s);
+    g.step_z(tasks, nt, j, 1, 1, true, false, s);
     if (W.with_k)
       hipLaunchKernelGGL(k_adj_kgrad, dim3(gk), dim3(256), 0, s, tasks, W.pairs, W.npair, j, g.n1,
                          g.n2, g.n3, g.zs->zw);
@@ -2008,6 +2020,7 @@ void run_adj_sweeps(const System& S, hipStream_t s) {
   W.npair = A.npair;
   W.max_ns = S.max_ns;
   W.with_k = A.with_k;
+  W.half_z = sym_half(S.g.sym);
   W.K = S.ck_stride;
   if (W.K > 0) {
     W.nround = S.ck.nround;
@@ -2325,6 +2338,8 @@ void build_adj_group(AdjGroup& G) {
   G.W.npair = (int)hp.size();
   G.W.max_ns = max_ns;
   G.W.with_k = G.with_k;
+  G.W.half_z = true;
+  for (System* S : G.sys) G.W.half_z = G.W.half_z && sym_half(S->g.sym);
   G.W.K = K;
   if (K > 0) {
     // round r of a system past its own rounds: recomputation skipped, adjoint
@@ -2538,6 +2553,7 @@ struct BatchInst {
 
 struct Group {
   int n1 = 0, n2 = 0, n3 = 0, np = 0;
+  bool half_z = true;            // every member's planes allow it (Grid::step_z)
   std::vector<int> members;
   // the members' chain-discretisation generations when the tasks were
   // copied: a restart (startup, set_checkpoint) frees the slabs the tasks
@@ -2596,6 +2612,7 @@ void build_groups(Batch& Bt) {
       G->n3 = S.g.n3;
       G->np = S.g.np;
     }
+    G->half_z = G->half_z && sym_half(S.g.sym);
     G->members.push_back(i);
     G->gen_start.push_back(S.gen_start);
     for (const auto& t : S.h_tasks) {
@@ -2624,7 +2641,7 @@ void batch_density(Batch& Bt, bool with_stress) {
     const Grid& g = Bt.inst[G.members[0]].S->g;
     if (!G.exec) {
       HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-      run_sweeps(g, G.tasks.p, (int)G.h_tasks.size(), G.max_ns, s);
+      run_sweeps(g, G.tasks.p, (int)G.h_tasks.size(), G.max_ns, G.half_z, s);
       HIPCHK(hipStreamEndCapture(s, &G.graph));
       HIPCHK(hipGraphInstantiate(&G.exec, G.graph, nullptr, nullptr, 0));
     }
@@ -2970,7 +2987,7 @@ int pscf_step_exp(int64_t step, const double* q_in, double* q_out) {
     t.C = S.abc.p + 2 * g.mc;
     t.q1 = S.q1.p;
     HIPCHK(hipMemcpyAsync(S.task.p, &t, sizeof t, hipMemcpyHostToDevice, S.st.s));
-    run_sweeps(g, S.task.p, 1, 1, S.st.s);
+    run_sweeps(g, S.task.p, 1, 1, false, S.st.s);
     hipLaunchKernelGGL(k_unpack, dim3(grid_blocks(g.m)), dim3(NTA), 0, S.st.s, S.slab.p + g.m, g.m, 1,
                        g.n1, g.n2, S.q1.p);
     HIPCHK(hipMemcpyAsync(q_out, S.q1.p, sizeof(double) * g.m, hipMemcpyDeviceToHost, S.st.s));
@@ -3035,7 +3052,7 @@ int pscf_step_exp_noalloc(const int ngrid[3], double ds, double b, const double*
     t.q1 = base + o_q1;
     StepTask* dtask = reinterpret_cast<StepTask*>(base);
     HIPCHK(hipMemcpyAsync(dtask, &t, sizeof t, hipMemcpyHostToDevice, s));
-    run_sweeps(g, dtask, 1, 1, s);
+    run_sweeps(g, dtask, 1, 1, false, s);
     hipLaunchKernelGGL(k_unpack, dim3(grid_blocks(g.m)), dim3(NTA), 0, s, t.slab + g.m, g.m, 1, g.n1, g.n2,
                        q_out);
     HIPCHK(hipGetLastError());
@@ -3079,7 +3096,7 @@ int pscf_profile_step_kernel(int64_t sys, int kind, int j, int reps, double* us)
       else if (kind == 2)
         g.step_c(S.tasks.p, S.ntask, j, false, s);
       else
-        g.step_z(S.tasks.p, S.ntask, j, kind == 1 ? 0 : 1, kind == 1 ? 2 : 1, false, s);
+        g.step_z(S.tasks.p, S.ntask, j, kind == 1 ? 0 : 1, kind == 1 ? 2 : 1, false, sym_half(g.sym), s);
     };
     launch();
     HIPCHK(hipEventRecord(S.ev[0], s));

@@ -97,3 +97,33 @@ def test_grouped_gradients(backend):
         sum((w.detach() / w[0].numel() * rho).sum() + Q.sum() for w, (rho, Q) in zip(ws, out)).backward()
         for w, ref in zip(ws, single):
             close(w.grad.cpu().numpy(), ref, 1e-11)
+
+
+I3 = (1, 0, 0, 0, 1, 0, 0, 0, 1)
+INV = ((-1, 0, 0, 0, -1, 0, 0, 0, -1), (0, 0, 0))
+CENTRED = {"body": [INV, (I3, (.5, .5, .5))], "A": [(I3, (0, .5, .5))], "B": [INV, (I3, (.5, 0, .5))],
+           "half edge": [(I3, (0, 0, .5))]}
+
+
+@pytest.mark.parametrize("grid", [(12, 16, 16), (16, 12, 24), (16, 24, 32)], ids=lambda g: "%dx%dx%d" % g)
+@pytest.mark.parametrize("name", list(CENTRED))
+def test_centred_planes(name, grid, backend):
+    """Translations along z: the z lines of half the edge, with even or odd kz."""
+    lib = get_lib(backend)
+    cell = ("orthorhombic", [2.0, 2.4, 2.2])
+    S, P = make(cell, CENTRED[name], grid, lib, 0), make(cell, [], grid, lib, 0)
+    rng = np.random.default_rng(31)
+    stars = np.zeros((2, S.N_star))
+    stars[:, :14] = rng.normal(0.0, 1.0, (2, 14))
+    rho, q, _ = S.density(stars)
+    got = S.grids()[1]
+    points = [(c, d, p) for c in (0, 1) for d in (1, -1) for p in (1, 4)]
+    qs = [S.q(*p) for p in points]
+    w = adjoint.stars_to_grid(S, torch.tensor(stars, device=lib.tensor_device)).detach()
+    want, Q = adjoint.density(P, w)
+    close(got, want.cpu().numpy())
+    close(q, Q.cpu().numpy())
+    for p, v in zip(points, qs):
+        close(v, P.q(*p))
+    many = S.density_many(np.stack([stars, 0.5 * stars]))
+    assert np.array_equal(many[0][0], rho)
